@@ -290,4 +290,15 @@ constexpr int kIslandB = 17, kIslandC = 128, kIslandJ = 3, kIslandR = 16;
 constexpr int kIslandS = kBlock == 64 ? 4 : 1;
 hipError_t launch_island_step(const DModel& d, const Launch& L, bool multi, dim3 grid, size_t lds, hipStream_t st);
 
+// The step for any dimensions with a fixed number of worlds per wave (b2_waves.hpp), per n_steps > 1 and plain model
+// (revolute joints only, no edge shapes, the v2.4.1 revolute solver).
+hipError_t launch_step_w1(const DModel& d, const Launch& L, bool multi, bool plain, dim3 grid, size_t lds,
+                          hipStream_t st);
+hipError_t launch_step_w2(const DModel& d, const Launch& L, bool multi, bool plain, dim3 grid, size_t lds,
+                          hipStream_t st);
+hipError_t launch_step_w4(const DModel& d, const Launch& L, bool multi, bool plain, dim3 grid, size_t lds,
+                          hipStream_t st);
+hipError_t launch_step_w8(const DModel& d, const Launch& L, bool multi, bool plain, dim3 grid, size_t lds,
+                          hipStream_t st);
+
 }  // namespace goi

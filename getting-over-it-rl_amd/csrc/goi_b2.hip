@@ -658,36 +658,38 @@ static size_t workspace_bytes(int B, int C, int J, int R) {
     return (size_t)Workspace::layout(B, C, J, R).words * sizeof(int);
 }
 
-// Worlds per 64-lane wavefront. One lane runs one world's whole step (a long serial chain of dependent work), so
-// a launch wants at least a few wavefronts per SIMD (256 CUs x 4 SIMDs) even when that leaves lanes idle.
-// GOI_WORLDS_PER_WAVE overrides (1..64).
+// Blocks of `lds` bytes of dynamic LDS that a CU holds at once: at most kBlocksPerCu (the register budget), and as many
+// as its 160 KB of LDS hold.
+static long blocks_per_cu(size_t lds) {
+    return std::min<long>(kBlocksPerCu, (long)(kCuLdsBytes / (lds + kStaticLdsBytes)));
+}
+
+// Worlds per 64-lane wavefront; GOI_WORLDS_PER_WAVE overrides (1..64). A launch ends with its slowest wave, and a wave
+// runs the paths of all its worlds one after another where they differ, while fewer worlds per wave give each world
+// more lanes: so the launch takes the smallest power of two whose blocks all fit the GPU at once (a second round of
+// blocks costs more than a larger wave: 4,096 rig worlds take 491 us at 1 a wave, two rounds, 343 at 2 and 360 at 4;
+// 8,192 worlds 693 at 1, 408 at 4 and 447 at 8; 16,320 worlds 857 at 4, two rounds, 455 at 8).
+//
+// Batches too large for that take the wave size with the most worlds resident per CU (blocks per CU x worlds per
+// block), the smaller on a tie: a CU's 160 KB of LDS can hold fewer than 8 blocks when the worlds' workspaces are
+// large. The 4-body rig with 40 slots: 8 worlds per wave, 8 blocks per CU. The rig with 12 boxes and 128 slots: 4
+// worlds per wave (30.6 KB, 5 blocks per CU: 20 worlds) rather than 8 (61 KB, 2 blocks: 16 worlds), measured 35%
+// faster at 65536 worlds.
 static int worlds_per_wave(int n, size_t ws_bytes_per_world) {
     const char* e = getenv("GOI_WORLDS_PER_WAVE");  // read per call: tests vary it within one process
     int forced = e ? atoi(e) : 0;
     if (forced < 0 || forced > kBlock) forced = 0;
     if (forced > 0)
         return std::min<long>(forced, std::max<long>(1, (kMaxLdsBytes - kBlock * sizeof(int)) / ws_bytes_per_world));
-    // Fewer worlds per wave fill more SIMDs, shrink the slowest lane a wave waits for and give each world more lanes
-    // in the block-cooperative passes, but past the waves a SIMD can hold (k_step's register budget allows two) the
-    // launch needs a second round. Measured at 16384 worlds of the 4-body rig, two waves per SIMD: 16 -> 1.32 ms,
-    // 8 -> 1.25 (one wave per SIMD: 32 -> 1.56, 16 -> 1.48). Aim for two waves per SIMD (8 per CU).
-    //
-    // A CU's 160 KB of LDS can hold fewer blocks than that when the worlds' workspaces are large, so among the wave
-    // sizes that fit, take the one with the most worlds resident per CU (blocks per CU x worlds per block), the
-    // smaller on a tie (more lanes per world). The 4-body rig with 40 slots: 8 worlds per wave, 8 blocks per CU. The
-    // rig with 12 boxes and 128 slots: 4 worlds per wave (30.6 KB, 5 blocks per CU: 20 worlds) rather than 8 (61 KB,
-    // 2 blocks: 16 worlds), measured 35% faster at 65536 worlds.
-    int top = kBlock;
-    while (top > 1 && (long)n / top < 8L * cu_count()) top /= 2;
     int wpw = 0;
     long best = -1;
-    for (int w = top; w >= 1; w /= 2) {
+    for (int w = 1; w <= kBlock; w *= 2) {
         const size_t lds = ws_bytes_per_world * w + kBlock * sizeof(int);
-        if (lds > kMaxLdsBytes) continue;
-        const long blocks = std::min<long>(kBlocksPerCu, (long)(kCuLdsBytes / (lds + kStaticLdsBytes)));
-        const long resident = blocks * w;
-        if (resident >= best) {  // >=: the smaller wave wins a tie
-            best = resident;
+        if (lds > kMaxLdsBytes) break;
+        const long blocks = blocks_per_cu(lds);
+        if (((long)n + w - 1) / w <= blocks * cu_count()) return w;
+        if (blocks * w > best) {  // >: the smaller wave wins a tie
+            best = blocks * w;
             wpw = w;
         }
     }
@@ -787,6 +789,18 @@ static int check_step_args(const GoiModel* model, const GoiStateView* state, con
     return GOI_OK;
 }
 
+// The step instance compiled for wpw worlds per wave, or null: k_step takes the other wave sizes (a forced odd one; 16
+// and above, for worlds with so few slots that a CU's LDS holds more of them that way) and launches with debug arrays.
+using WaveLaunch = hipError_t (*)(const DModel&, const Launch&, bool, bool, dim3, size_t, hipStream_t);
+static WaveLaunch wave_instance(int wpw) {
+#ifdef GOI_HOST_BUILD
+    return wpw == 1 ? launch_step_w1 : nullptr;  // one lane per block
+#else
+    return wpw == 1 ? launch_step_w1 : wpw == 2 ? launch_step_w2 : wpw == 4 ? launch_step_w4
+         : wpw == 8 ? launch_step_w8 : nullptr;
+#endif
+}
+
 // Launches n_steps steps of every world of `state` with the constraint rows at `rows` (scratch_words(state) words).
 // order_buf: room for the block order (pitch + 64 words), or null (the blocks then run in the XCD order). A launch
 // whose blocks do not all fit on the GPU at once, with TOI on, first orders its blocks (k_group_order).
@@ -805,7 +819,7 @@ static int launch_step(const GoiModel* M, const GoiStateView* state, const GoiSe
     // the fixed instances write no debug arrays (it frees the scalar registers their pointers would hold)
     const GoiDebug& D = L.dbg;
     const bool dbg = D.body_island || D.contact_island || D.contact_order || D.n_islands || D.toi_event_slot ||
-                     D.toi_event_alpha || D.toi_event_island || D.toi_island_rows;
+                     D.toi_event_alpha || D.toi_event_island || D.toi_island_rows || D.status;
     const bool rig = L.B == kRigB && L.C == kRigC && L.J == kRigJ && L.R == kRigR && L.wpw == kRigS &&
                      M->d.B == kRigB && M->d.J == kRigJ && M->d.R == kRigR && L.packed && !dbg;
     const dim3 g(grid), b(kBlock);
@@ -815,7 +829,7 @@ static int launch_step(const GoiModel* M, const GoiStateView* state, const GoiSe
                         L.packed && plain && !dbg;
     g_last_launch = GoiLaunchInfo{L.wpw, grid, (int32_t)lds,
                                   rig ? GOI_KERNEL_RIG : island ? GOI_KERNEL_ISLAND : GOI_KERNEL_GENERIC};
-    const long resident = (long)cu_count() * std::min<long>(kBlocksPerCu, (long)(kCuLdsBytes / (lds + kStaticLdsBytes)));
+    const long resident = (long)cu_count() * blocks_per_cu(lds);
     if (order_buf && settings->continuous_physics && grid > resident) {
         int* cost = order_buf + state->pitch + 64;
         hipLaunchKernelGGL(k_group_order, dim3(1), dim3(kBlock), 0, st,
@@ -831,6 +845,9 @@ static int launch_step(const GoiModel* M, const GoiStateView* state, const GoiSe
     } else if (island) {
         const hipError_t e = launch_island_step(M->d, L, n_steps != 1, g, lds, st);
         if (e != hipSuccess) return fail(GOI_E_HIP, std::string("launch_island_step: ") + hipGetErrorString(e));
+    } else if (!dbg && wave_instance(L.wpw)) {
+        const hipError_t e = wave_instance(L.wpw)(M->d, L, n_steps != 1, plain, g, lds, st);
+        if (e != hipSuccess) return fail(GOI_E_HIP, std::string("launch_step_w: ") + hipGetErrorString(e));
     } else if (n_steps == 1) {
         hipLaunchKernelGGL(k_step<false>, g, b, lds, st, M->d, L);
     } else {

@@ -1,0 +1,11 @@
+// goi_b2_w4.hip - the step for any dimensions, 4 worlds per wave (b2_waves.hpp).
+#include "b2_waves.hpp"
+
+namespace goi {
+
+hipError_t launch_step_w4(const DModel& d, const Launch& L, bool multi, bool plain, dim3 grid, size_t lds,
+                          hipStream_t st) {
+    return launch_wave_instance<4>(d, L, multi, plain, grid, lds, st);
+}
+
+}  // namespace goi

@@ -1,0 +1,62 @@
+"""The step instances compiled for 1, 2, 4 and 8 worlds per wave (any dimensions, any State layout) and the rule that
+picks the wave size, against the oracle bit for bit."""
+import numpy as np
+import pytest
+
+from util import b2, leaf_mismatches, perturbed
+import scene_defs
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+def _compare(model, state, settings, dt, launches, oracle, n_steps=1, pitch=None, nan_equal=False):
+    dev, ref = b2.layout.to_device(state, "cuda", pitch), oracle.copy(state)
+    for k in range(launches):
+        b2.step_n_(model, dev, settings, dt, n_steps)
+        for _ in range(n_steps):
+            oracle.step_(model, ref, settings, dt)
+        bad = leaf_mismatches(ref, b2.layout.to_host(dev), nan_equal)
+        assert bad == [], f"launch {k + 1}: {bad[:4]}"
+    return ref
+
+
+@pytest.mark.parametrize("wpw", [1, 2, 4, 8])
+@pytest.mark.parametrize("case", ["quad_41", "native", "joints", "pile", "full"])
+def test_wave_instances_parity(oracle, monkeypatch, case, wpw):
+    """Each wave size's instances, plain and not, single- and multi-step: 61 worlds (the last block partly filled
+    except at 1 a wave) of the rig with an odd slot count, the rig on a native chain, every joint type (the general
+    joint rows), box piles, and a State in the full fixture layout; stock settings, then the v2.3.1 revolute solver."""
+    from dataclasses import replace
+    monkeypatch.setenv("GOI_WORLDS_PER_WAVE", str(wpw))
+    n, dt = 61, 1.0 / 60.0
+    if case in ("quad_41", "native"):
+        s, m, st, cfg = b2.scenes.make_config(4, n, edges="native" if case == "native" else "quad",
+                                              capacity=41 if case == "quad_41" else None)
+        dt = cfg.dt
+    elif case == "full":
+        cfg = b2.scenes.CONFIGS[4]
+        s = b2.scenes.settings_for(cfg)
+        m, one, pts = b2.scenes.build_world(cfg, s)
+        st, dt = b2.scenes.place_worlds(cfg, m, one, pts, n), cfg.dt
+    else:
+        s, m, one = scene_defs.build_test_scene(case, iterations=(8, 3))
+        st = perturbed(one, n)
+    for settings in (s, replace(s, revolute_v24=False)):
+        ref = _compare(m, st, settings, dt, 6, oracle)
+        ref = _compare(m, ref, settings, dt, 2, oracle, n_steps=3)
+        assert b2.last_launch()["worlds_per_wave"] == wpw
+
+
+@pytest.mark.parametrize("n", [1, 2047, 2048, 2049, 4097, 8193, 16383, 16384, 16385])
+def test_wave_size_rule(oracle, n):
+    """The smallest wave size whose blocks all fit the GPU at once (8 blocks a CU for the rig), the most resident one
+    above that; two steps at the edges of each range."""
+    s, m, st, cfg = b2.scenes.make_config(4, min(n, 256))
+    idx = np.arange(n) % min(n, 256)
+    st = b2.world.from_leaves([np.ascontiguousarray(x[idx]) for x in b2.world.leaves(st)])
+    _compare(m, st, s, cfg.dt, 2, oracle)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    info = b2.last_launch()
+    want = next((w for w in (1, 2, 4, 8) if -(-n // w) <= 8 * cus), 8)
+    assert info["worlds_per_wave"] == want and info["blocks"] == -(-n // want), info
