@@ -142,8 +142,7 @@ GOI_D void jn_prepare(const DModel& m, const World& W, const Bodies& bd, const R
 }
 
 // the velocity part of InitVelocityConstraints (joints.py:202-248)
-template <class BD>
-GOI_D void jn_warm_start(const BD& bd, const Rows& R, int i, bool v24, bool rev_only) {
+GOI_D void jn_warm_start(const Bodies& bd, const Rows& R, int i, bool v24, bool rev_only) {
     const int type = rev_only ? (int)GOI_REVOLUTE : R.geti(i, JF_TYPE), ia = R.geti(i, JF_IA), ib = R.geti(i, JF_IB);
     const float mA = R.getf(i, JF_MA), mB = R.getf(i, JF_MB), iA = R.getf(i, JF_IIA), iB = R.getf(i, JF_IIB);
     const float ix = R.getf(i, JF_IMP0), iy = R.getf(i, JF_IMP1), iz = R.getf(i, JF_IMP2), mi = R.getf(i, JF_MIMP);
@@ -178,8 +177,7 @@ GOI_D void jn_warm_start(const BD& bd, const Rows& R, int i, bool v24, bool rev_
 }
 
 // SolveVelocityConstraints for joint row i (joints.py:257-437, revolute24.patch:166-240)
-template <class BD>
-GOI_D void jn_solve_velocity(const BD& bd, const Rows& R, int i, bool v24, bool rev_only) {
+GOI_D void jn_solve_velocity(const Bodies& bd, const Rows& R, int i, bool v24, bool rev_only) {
     const int type = rev_only ? (int)GOI_REVOLUTE : R.geti(i, JF_TYPE), ia = R.geti(i, JF_IA), ib = R.geti(i, JF_IB);
     const float mA = R.getf(i, JF_MA), mB = R.getf(i, JF_MB), iA = R.getf(i, JF_IIA), iB = R.getf(i, JF_IIB);
     const bool emotor = R.geti(i, JF_EMOTOR) != 0, elimit = R.geti(i, JF_ELIMIT) != 0;
@@ -329,33 +327,81 @@ GOI_D void jn_solve_velocity(const BD& bd, const Rows& R, int i, bool v24, bool 
     bd.set_v(ib, vB, wB);
 }
 
-// A revolute joint's velocity-solve fields for the v2.4.1 solver (revolute24.patch:166-240), loaded in one batch.
-// A revolute-only model's joint passes load joint i + 1's row while joint i is solved (rev_velocity_sweep); the
-// operations are those of jn_solve_velocity's v2.4.1 revolute branch.
-struct RevVRow {
-    int ia, ib;
+// A revolute joint's row under the v2.4.1 solver (revolute24.patch:78-330, joints.py:61-520), set up by the lane that
+// keeps it in registers through the velocity and position iterations: the operations of jn_prepare, jn_warm_start,
+// jn_solve_velocity and jn_solve_position's v2.4.1 revolute branches. inv_det is solve22's reciprocal determinant, the
+// same in every iteration. The z impulse (the 2.3.1 solver's) stays as the State holds it.
+struct RevRow {
+    int jid, ia, ib, state, isl;
     bool emotor, elimit;
-    float mA, mB, iA, iB, k11, k12, k21, k22, i0, i1, i3, i4, mi, maximp, mspeed, mmass, angle, inv_dt, lower, upper;
-    V2 rA, rB;
+    float mA, mB, iA, iB, k11, k12, k21, k22, inv_det, i0, i1, i3, i4, mi, maximp, mspeed, mmass, angle, inv_dt;
+    float lower, upper, ref;
+    V2 rA, rB, la, lb;
 };
-GOI_D RevVRow load_rev_vrow(const Rows& R, int i) {
-    RevVRow r;
-    r.ia = R.geti(i, JF_IA); r.ib = R.geti(i, JF_IB);
-    r.emotor = R.geti(i, JF_EMOTOR) != 0; r.elimit = R.geti(i, JF_ELIMIT) != 0;
-    r.mA = R.getf(i, JF_MA); r.mB = R.getf(i, JF_MB); r.iA = R.getf(i, JF_IIA); r.iB = R.getf(i, JF_IIB);
-    r.k11 = R.getf(i, JF_EXX); r.k21 = R.getf(i, JF_EXX + 1); r.k12 = R.getf(i, JF_EYX); r.k22 = R.getf(i, JF_EYX + 1);
-    r.i0 = R.getf(i, JF_IMP0); r.i1 = R.getf(i, JF_IMP1); r.i3 = R.getf(i, JF_IMP3); r.i4 = R.getf(i, JF_IMP4);
-    r.mi = R.getf(i, JF_MIMP);
-    r.maximp = R.getf(i, JF_MAXIMP); r.mspeed = R.getf(i, JF_MSPEED); r.mmass = R.getf(i, JF_MMASS);
-    r.rA = R.get2(i, JF_RA); r.rB = R.get2(i, JF_RB);
-    r.angle = R.getf(i, JF_ANGLE); r.inv_dt = R.getf(i, JF_INVDT);
-    r.lower = R.getf(i, JF_LOWER); r.upper = R.getf(i, JF_UPPER);
+GOI_D RevRow rev_row_of(const DModel& m, const World& W, const Bodies& bd, int jid, const GoiSettings& s, float dt,
+                        float dt_ratio, bool warm) {
+    const MJoint j = m.joint[jid];
+    RevRow r;
+    r.jid = jid; r.ia = j.a; r.ib = j.b;
+    r.emotor = W.u8(GOI_J_ENABLE_MOTOR, jid) != 0; r.elimit = W.u8(GOI_J_ENABLE_LIMIT, jid) != 0;
+    r.lower = W.f(GOI_J_LOWER, jid); r.upper = W.f(GOI_J_UPPER, jid); r.ref = j.reference_angle;
+    const float ix = W.f(GOI_J_IMPULSE, 3 * jid), iy = W.f(GOI_J_IMPULSE, 3 * jid + 1);
+    float mimp = W.f(GOI_J_MOTOR_IMPULSE, jid);
+    const float lo_in = W.f(GOI_J_LOWER_IMPULSE, jid), up_in = W.f(GOI_J_UPPER_IMPULSE, jid);
+    r.mspeed = W.f(GOI_J_MOTOR_SPEED, jid);
+    r.maximp = dt * W.f(GOI_J_MAX_MOTOR, jid);
+    r.inv_dt = dt > 0.0f ? 1.0f / dt : 0.0f;
+    r.mA = W.f(GOI_B_INV_MASS, r.ia); r.mB = W.f(GOI_B_INV_MASS, r.ib);
+    r.iA = W.f(GOI_B_INV_INERTIA, r.ia); r.iB = W.f(GOI_B_INV_INERTIA, r.ib);
+    Rot qA, qB;
+    qA.c = bd.at(6, r.ia); qA.s = bd.at(7, r.ia);
+    qB.c = bd.at(6, r.ib); qB.s = bd.at(7, r.ib);
+    r.la = j.anchor_a - W.v2(GOI_B_LOCAL_CENTER, r.ia);
+    r.lb = j.anchor_b - W.v2(GOI_B_LOCAL_CENTER, r.ib);
+    const V2 rA = mul(qA, r.la), rB = mul(qB, r.lb);
+    r.rA = rA; r.rB = rB;
+    const float mA = r.mA, mB = r.mB, iA = r.iA, iB = r.iB;
+    r.k11 = ((mA + mB) + rA.y * rA.y * iA) + rB.y * rB.y * iB;
+    r.k12 = -rA.y * rA.x * iA - rB.y * rB.x * iB;
+    r.k21 = r.k12;
+    r.k22 = ((mA + mB) + rA.x * rA.x * iA) + rB.x * rB.x * iB;
+    float det = r.k11 * r.k22 - r.k12 * r.k21;
+    if (det != 0.0f) det = fdiv(1.0f, det);
+    r.inv_det = det;
+    const bool fixed = (iA + iB) == 0.0f;
+    r.mmass = (iA + iB) > 0.0f ? 1.0f / (iA + iB) : 0.0f;
+    if (!r.emotor || fixed) mimp = 0.0f;
+    r.angle = (bd.a(r.ib) - bd.a(r.ia)) - r.ref;
+    const bool lim_on = r.elimit && !fixed;
+    r.state = !lim_on ? kInactive : babs(r.upper - r.lower) < 2.0f * s.angular_slop ? kEqual
+              : r.angle <= r.lower ? kAtLower : r.angle >= r.upper ? kAtUpper : kInactive;
+    const float lo = lim_on ? lo_in : 0.0f, up = lim_on ? up_in : 0.0f;
+    r.i0 = warm ? ix * dt_ratio : 0.0f;
+    r.i1 = warm ? iy * dt_ratio : 0.0f;
+    r.i3 = warm ? lo * dt_ratio : 0.0f;
+    r.i4 = warm ? up * dt_ratio : 0.0f;
+    r.mi = warm ? mimp * dt_ratio : 0.0f;
     return r;
 }
-template <class BD>
-GOI_D void solve_rev_vrow(const BD& bd, RevVRow& r) {
-    V2 vA = bd.v(r.ia), vB = bd.v(r.ib);
-    float wA = bd.w(r.ia), wB = bd.w(r.ib);
+GOI_D void warm_rev_row(const LaneBodies& bd, const RevRow& r) {
+    const V2 vA0 = bd.v(r.ia), vB0 = bd.v(r.ib);
+    const float wA0 = bd.w(r.ia), wB0 = bd.w(r.ib);
+    V2 vA = vA0, vB = vB0;
+    float wA = wA0, wB = wB0;
+    const V2 P = mk(r.i0, r.i1);
+    vA = vA - r.mA * P;
+    vB = vB + r.mB * P;
+    const float axial = (r.mi + r.i3) - r.i4;
+    wA = wA - r.iA * (cross(r.rA, P) + axial);
+    wB = wB + r.iB * (cross(r.rB, P) + axial);
+    bd.set_v(r.ia, vA, wA, vA0, wA0);
+    bd.set_v(r.ib, vB, wB, vB0, wB0);
+}
+GOI_D void solve_rev_row(const LaneBodies& bd, RevRow& r) {
+    const V2 vA0 = bd.v(r.ia), vB0 = bd.v(r.ib);
+    const float wA0 = bd.w(r.ia), wB0 = bd.w(r.ib);
+    V2 vA = vA0, vB = vB0;
+    float wA = wA0, wB = wB0;
     const float mA = r.mA, mB = r.mB, iA = r.iA, iB = r.iB;
     const bool fixed = (iA + iB) == 0.0f;
     if (r.emotor && !fixed) {
@@ -382,39 +428,37 @@ GOI_D void solve_rev_vrow(const BD& bd, RevVRow& r) {
         wA = wA + iA * impulse;
         wB = wB - iB * impulse;
     }
-    const V2 p = solve22(r.k11, r.k12, r.k21, r.k22, -rel_vel(vB, wB, r.rB, vA, wA, r.rA));
+    const V2 b = -rel_vel(vB, wB, r.rB, vA, wA, r.rA);
+    const V2 p = mk(r.inv_det * (r.k22 * b.x - r.k12 * b.y), r.inv_det * (r.k11 * b.y - r.k21 * b.x));
     r.i0 = r.i0 + p.x;
     r.i1 = r.i1 + p.y;
     vA = vA - mA * p; wA = wA - iA * cross(r.rA, p);
     vB = vB + mB * p; wB = wB + iB * cross(r.rB, p);
-    bd.set_v(r.ia, vA, wA);
-    bd.set_v(r.ib, vB, wB);
+    bd.set_v(r.ia, vA, wA, vA0, wA0);
+    bd.set_v(r.ib, vB, wB, vB0, wB0);
 }
-// the impulses the solve changes (the revolute v2.4.1 branch leaves impulse z as it is)
-GOI_D void store_rev_impulses(const Rows& R, int i, const RevVRow& r) {
-    R.setf(i, JF_IMP0, r.i0); R.setf(i, JF_IMP1, r.i1);
-    R.setf(i, JF_IMP3, r.i3); R.setf(i, JF_IMP4, r.i4); R.setf(i, JF_MIMP, r.mi);
+GOI_D void store_rev_row(const World& W, const RevRow& r) {
+    const int j = r.jid;
+    W.f(GOI_J_IMPULSE, 3 * j) = r.i0;
+    W.f(GOI_J_IMPULSE, 3 * j + 1) = r.i1;
+    W.f(GOI_J_MOTOR_IMPULSE, j) = r.mi;
+    W.i32(GOI_J_LIMIT_STATE, j) = r.state;
+    W.f(GOI_J_LOWER_IMPULSE, j) = r.i3;
+    W.f(GOI_J_UPPER_IMPULSE, j) = r.i4;
 }
-// joint rows i0..n-1 of a revolute-only model under the v2.4.1 solver, once each, in order
-template <class BD>
-GOI_D void rev_velocity_sweep(const BD& bd, const Rows& R, int i0, int n) {
-    if (n <= i0) return;
-    RevVRow a = load_rev_vrow(R, i0), b;
-    for (int i = i0; i < n; i += 2) {  // as cs_solve_velocity_sweep: joint i + 1 in flight while joint i is solved
-        if (i + 1 < n) b = load_rev_vrow(R, i + 1);
-        solve_rev_vrow(bd, a);
-        store_rev_impulses(R, i, a);
-        if (i + 1 >= n) break;
-        if (i + 2 < n) a = load_rev_vrow(R, i + 2);
-        solve_rev_vrow(bd, b);
-        store_rev_impulses(R, i + 1, b);
-    }
+// the row's position-solver fields as row i of the row tile (jn_solve_position's)
+GOI_D void store_rev_prow(const Rows& R, int i, const RevRow& r) {
+    R.seti(i, JF_JID, r.jid); R.seti(i, JF_TYPE, (int)GOI_REVOLUTE); R.seti(i, JF_IA, r.ia); R.seti(i, JF_IB, r.ib);
+    R.setf(i, JF_MA, r.mA); R.setf(i, JF_MB, r.mB); R.setf(i, JF_IIA, r.iA); R.setf(i, JF_IIB, r.iB);
+    R.seti(i, JF_ELIMIT, r.elimit); R.seti(i, JF_STATE, r.state); R.setf(i, JF_MMASS, r.mmass);
+    R.setf(i, JF_LOWER, r.lower); R.setf(i, JF_UPPER, r.upper); R.setf(i, JF_REF, r.ref);
+    R.set2(i, JF_LA, r.la); R.set2(i, JF_LB, r.lb);
 }
 
-// the point part of the revolute position solve (joints.py:501-520)
+// the point part of the revolute position solve (joints.py:501-520); qA, qB the rotations of aA and aB
 GOI_D bool rev_point(float mA, float mB, float iA, float iB, V2 la, V2 lb, V2& cA, float& aA, V2& cB, float& aB,
-                     float ang_err, const GoiSettings& s) {
-    const V2 rA = mul(rot_of(aA), la), rB = mul(rot_of(aB), lb);
+                     Rot qA, Rot qB, float ang_err, const GoiSettings& s) {
+    const V2 rA = mul(qA, la), rB = mul(qB, lb);
     const V2 C = ((cB + rB) - cA) - rA;
     const float pos_err = length(C);
     const float kxx = ((mA + mB) + iA * rA.y * rA.y) + iB * rB.y * rB.y;
@@ -426,9 +470,51 @@ GOI_D bool rev_point(float mA, float mB, float iA, float iB, V2 la, V2 lb, V2& c
     return pos_err <= s.linear_slop && ang_err <= s.angular_slop;
 }
 
+// the limit part of the revolute position solve under the v2.4.1 solver; returns its angular error
+GOI_D float rev_limit_v24(float iA, float iB, float mmass, float lower, float upper, float ref, float& aA, float& aB,
+                          const GoiSettings& s) {
+    const float mac = s.max_angular_correction;
+    const float angle = (aB - aA) - ref;
+    float C = 0.0f;
+    if (babs(upper - lower) < 2.0f * s.angular_slop) C = bclamp(angle - lower, -mac, mac);
+    else if (angle <= lower) C = bclamp((angle - lower) + s.angular_slop, -mac, 0.0f);
+    else if (angle >= upper) C = bclamp((angle - upper) - s.angular_slop, 0.0f, mac);
+    const float li = -mmass * C;
+    aA = aA - iA * li;
+    aB = aB + iB * li;
+    return babs(C);
+}
+
+// jn_solve_position of a RevRow. Two neighbouring lanes hold the same row where `pair` is set: each takes the sin/cos
+// of one body's angle and they exchange them (a double-precision evaluation is about 40 of the row's 150 instructions).
+GOI_D bool solve_rev_position(const LaneBodies& bd, const RevRow& r, const GoiSettings& s, bool pair, bool odd) {
+    const V2 cA0 = bd.c(r.ia), cB0 = bd.c(r.ib);
+    const float aA0 = bd.a(r.ia), aB0 = bd.a(r.ib);
+    V2 cA = cA0, cB = cB0;
+    float aA = aA0, aB = aB0;
+    float ang_err = 0.0f;
+    if (r.elimit && (r.iA + r.iB) != 0.0f)
+        ang_err = rev_limit_v24(r.iA, r.iB, r.mmass, r.lower, r.upper, r.ref, aA, aB, s);
+    Rot qA, qB;
+    if (pair) {
+        const Rot mine = rot_of(odd ? aB : aA);
+        Rot other;
+        other.c = lane_partner(mine.c, 1);
+        other.s = lane_partner(mine.s, 1);
+        qA = odd ? other : mine;
+        qB = odd ? mine : other;
+    } else {
+        qA = rot_of(aA);
+        qB = rot_of(aB);
+    }
+    const bool ok = rev_point(r.mA, r.mB, r.iA, r.iB, r.la, r.lb, cA, aA, cB, aB, qA, qB, ang_err, s);
+    bd.set_c(r.ia, cA, aA, cA0, aA0);
+    bd.set_c(r.ib, cB, aB, cB0, aB0);
+    return ok;
+}
+
 // SolvePositionConstraints for joint row i (joints.py:462-606); returns the joint's ok flag
-template <class BD>
-GOI_D bool jn_solve_position(const BD& bd, const Rows& R, int i, const GoiSettings& s, bool rev_only) {
+GOI_D bool jn_solve_position(const Bodies& bd, const Rows& R, int i, const GoiSettings& s, bool rev_only) {
     const int type = rev_only ? (int)GOI_REVOLUTE : R.geti(i, JF_TYPE), ia = R.geti(i, JF_IA), ib = R.geti(i, JF_IB);
     const float mA = R.getf(i, JF_MA), mB = R.getf(i, JF_MB), iA = R.getf(i, JF_IIA), iB = R.getf(i, JF_IIB);
     const bool elimit = R.geti(i, JF_ELIMIT) != 0;
@@ -446,17 +532,7 @@ GOI_D bool jn_solve_position(const BD& bd, const Rows& R, int i, const GoiSettin
         const float mmass = jmmass;
         float ang_err = 0.0f;
         if (s.revolute_v24) {
-            if (elimit && !fixed) {
-                const float angle = (aB - aA) - ref;
-                float C = 0.0f;
-                if (babs(upper - lower) < 2.0f * s.angular_slop) C = bclamp(angle - lower, -mac, mac);
-                else if (angle <= lower) C = bclamp((angle - lower) + s.angular_slop, -mac, 0.0f);
-                else if (angle >= upper) C = bclamp((angle - upper) - s.angular_slop, 0.0f, mac);
-                const float li = -mmass * C;
-                aA = aA - iA * li;
-                aB = aB + iB * li;
-                ang_err = babs(C);
-            }
+            if (elimit && !fixed) ang_err = rev_limit_v24(iA, iB, mmass, lower, upper, ref, aA, aB, s);
         } else {
             const int st = jst;
             if (elimit && st != kInactive && !fixed) {
@@ -481,7 +557,7 @@ GOI_D bool jn_solve_position(const BD& bd, const Rows& R, int i, const GoiSettin
                 aB = aB + iB * li;
             }
         }
-        ok = rev_point(mA, mB, iA, iB, jla, jlb, cA, aA, cB, aB, ang_err, s);
+        ok = rev_point(mA, mB, iA, iB, jla, jlb, cA, aA, cB, aB, rot_of(aA), rot_of(aB), ang_err, s);
     } else if (type == GOI_PRISMATIC) {
         const Rot qA = rot_of(aA), qB = rot_of(aB);
         const V2 rA = mul(qA, R.get2(i, JF_LA)), rB = mul(qB, R.get2(i, JF_LB));

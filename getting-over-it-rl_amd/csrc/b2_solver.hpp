@@ -31,30 +31,42 @@ struct Bodies {
     GOI_D V2 c(int b) const { return mk(cx(b), cy(b)); }
     GOI_D void set_v(int b, V2 x, float ww) const { vx(b) = x.x; vy(b) = x.y; w(b) = ww; }
     GOI_D void set_c(int b, V2 x, float aa) const { cx(b) = x.x; cy(b) = x.y; a(b) = aa; }
+    // the same with the values read before, which LaneBodies compares
+    GOI_D void set_v(int b, V2 x, float ww, V2, float) const { set_v(b, x, ww); }
+    GOI_D void set_c(int b, V2 x, float aa, V2, float) const { set_c(b, x, aa); }
+    GOI_D void note_sep(float) const {}
 };
 
-// One lane's view of the bodies while the lanes of a world's group solve its islands side by side, each lane its own
-// island (island.py:3-7: islands share no body but static ones). The island's bodies (`own`) are read and written;
-// another body that a row touches, a static one, is only read: Box2D's update of it (x - 0 * P) leaves it unchanged
-// unless an impulse is not finite or the value is -0, and a write that would change it raises the world's flag
-// (`changed`) instead, after which the world solves its islands again one after another. Without such a write, every
-// row saw the values it sees in Box2D's order, so the results are the same floats.
-struct IslandBodies {
+// The bodies as a lane sees them while the lanes of a world's group solve different rows at once (LaneContacts, RevRow).
+// No two of those rows share a body but static ones (`fixed`), which are only read: Box2D's update of a static body
+// (x - 0 * P) leaves it unchanged unless an impulse is not finite or the value is -0. A write that would change it, and
+// a separation that is NaN (the minimum over an island's rows then depends on their order), raise `changed` instead;
+// the world then runs the phase again row by row. Without either, every row saw the values it sees in Box2D's order,
+// so the results are the same floats.
+struct LaneBodies {
     Bodies bd;
-    unsigned long long own;
-    int* changed;
+    unsigned long long fixed;
+    unsigned* changed;  // nonzero: see above
     GOI_D V2 v(int b) const { return bd.v(b); }
     GOI_D float w(int b) const { return bd.w(b); }
     GOI_D V2 c(int b) const { return bd.c(b); }
     GOI_D float a(int b) const { return bd.a(b); }
-    GOI_D static bool differ(float x, float y) { return __float_as_uint(x) != __float_as_uint(y); }
-    GOI_D void set_v(int b, V2 x, float ww) const {
-        if ((own >> b) & 1ull) bd.set_v(b, x, ww);
-        else if (differ(x.x, bd.vx(b)) || differ(x.y, bd.vy(b)) || differ(ww, bd.w(b))) *changed = 1;
+    // a static body's write stores the value it has or raises `changed` (no branch: a branch costs more than the stores)
+    GOI_D void note(int b, V2 x, float s, V2 was, float was_s) const {
+        const auto bits = [](float p, float q) { return __float_as_uint(p) ^ __float_as_uint(q); };
+        const unsigned mask = 0u - (unsigned)((fixed >> b) & 1ull);
+        *changed |= mask & (bits(x.x, was.x) | bits(x.y, was.y) | bits(s, was_s));
     }
-    GOI_D void set_c(int b, V2 x, float aa) const {
-        if ((own >> b) & 1ull) bd.set_c(b, x, aa);
-        else if (differ(x.x, bd.cx(b)) || differ(x.y, bd.cy(b)) || differ(aa, bd.a(b))) *changed = 1;
+    GOI_D void set_v(int b, V2 x, float ww, V2 was, float was_w) const {
+        note(b, x, ww, was, was_w);
+        bd.set_v(b, x, ww);
+    }
+    GOI_D void set_c(int b, V2 x, float aa, V2 was, float was_a) const {
+        note(b, x, aa, was, was_a);
+        bd.set_c(b, x, aa);
+    }
+    GOI_D void note_sep(float sep) const {
+        if (sep != sep) *changed = 1u;
     }
 };
 
@@ -73,19 +85,6 @@ struct Islands {
     GOI_D int& body_island(int b) const { return W.bisl(b); }
     GOI_D int& contact_island(int c) const { return W.cisl(c); }
     GOI_D int& joint_island(int j) const { return W.jisl(j); }
-    // island k's contact rows [c0, c1) and joint rows [j0, j1) of the solve order (find_islands notes where each
-    // island's rows start)
-    GOI_D void rows_of(int k, int& c0, int& c1, int& j0, int& j1) const {
-        const int s0 = W.ibuf(k), s1 = k + 1 < n ? W.ibuf(k + 1) : (nc | (nj << 16));
-        c0 = s0 & 0xffff; j0 = s0 >> 16;
-        c1 = s1 & 0xffff; j1 = s1 >> 16;
-    }
-    GOI_D unsigned long long bodies_of(int k) const {
-        unsigned long long own = 0ull;
-        for (int b = 0; b < W.B; ++b)
-            if (body_island(b) == k) own |= 1ull << b;
-        return own;
-    }
 };
 
 // b2World::Solve's depth-first search: seeds newest body first; popping b wakes it, walks b's touching contacts
@@ -103,7 +102,6 @@ GOI_D void find_islands(const DModel& m, const World& W, Islands& I) {
         if ((bflag >> seed) & 1ull) continue;
         if (!W.awake(seed) || !W.active(seed) || W.is_static(seed)) continue;
         const int isl = nisl++;
-        if (m.island_lanes) W.ibuf(isl) = nc | (nj << 16);  // the island's first rows (nc <= 256, nj <= 64)
         int sp = 0;
         W.stack(sp++) = seed;
         bflag |= 1ull << seed;
@@ -151,43 +149,63 @@ GOI_D void find_islands(const DModel& m, const World& W, Islands& I) {
 
 // ---------------------------------------------------------------- contact solver (contact_solver.py)
 
-// b2ContactSolver constructor + InitializeVelocityConstraints for contact slot `slot` into row i
-// (contact_solver.py:32-147). Body positions/velocities from the LDS arrays; qA/qB the bodies' rotations.
-GOI_D void cs_prepare(const DModel& m, const World& W, const Bodies& bd, const Rows& R, int i, int slot, bool warm,
-                      float dt_ratio, Rot qA, Rot qB, float velocity_threshold) {
-    const int fa = W.fa(slot), fb = W.fb(slot);
-    const int ia = W.ba(slot), ib = W.bb(slot);
-    const float mA = W.f(GOI_B_INV_MASS, ia), mB = W.f(GOI_B_INV_MASS, ib);
-    const float iA = W.f(GOI_B_INV_INERTIA, ia), iB = W.f(GOI_B_INV_INERTIA, ib);
-    const V2 lcA = W.v2(GOI_B_LOCAL_CENTER, ia), lcB = W.v2(GOI_B_LOCAL_CENTER, ib);
-    const float radA = m.fix[fa].radius, radB = m.fix[fb].radius;
-    const int mtype = W.i32(GOI_C_MTYPE, slot);
-    const int cnt = W.ccount(slot);
-    const V2 ln = W.v2(GOI_C_LOCAL_NORMAL, slot), lp = W.v2(GOI_C_LOCAL_POINT, slot);
-    const V2 pl0 = W.v2(GOI_C_POINT_LOCAL, 2 * slot), pl1 = W.v2(GOI_C_POINT_LOCAL, 2 * slot + 1);
-    R.seti(i, CF_SLOT, slot); R.seti(i, CF_IA, ia); R.seti(i, CF_IB, ib);
-    R.seti(i, CF_PC_COUNT, cnt); R.seti(i, CF_MTYPE, mtype);
-    R.setf(i, CF_MA, mA); R.setf(i, CF_MB, mB); R.setf(i, CF_IIA, iA); R.setf(i, CF_IIB, iB);
-    R.set2(i, CF_LN, ln); R.set2(i, CF_LP, lp); R.set2(i, CF_PL0, pl0); R.set2(i, CF_PL1, pl1);
-    R.set2(i, CF_LCA, lcA); R.set2(i, CF_LCB, lcB); R.setf(i, CF_RADA, radA); R.setf(i, CF_RADB, radB);
-    R.setf(i, CF_NI0, warm ? dt_ratio * W.f(GOI_C_NORMAL_IMPULSE, 2 * slot) : 0.0f);
-    R.setf(i, CF_NI1, warm ? dt_ratio * W.f(GOI_C_NORMAL_IMPULSE, 2 * slot + 1) : 0.0f);
-    R.setf(i, CF_TI0, warm ? dt_ratio * W.f(GOI_C_TANGENT_IMPULSE, 2 * slot) : 0.0f);
-    R.setf(i, CF_TI1, warm ? dt_ratio * W.f(GOI_C_TANGENT_IMPULSE, 2 * slot + 1) : 0.0f);
-    R.setf(i, CF_FRICTION, W.f(GOI_C_FRICTION, slot));
-    R.setf(i, CF_TSPEED, W.f(GOI_C_TANGENT_SPEED, slot));
+// A contact row's velocity-solver fields, loaded in one batch (every field, whether or not the row's point count
+// uses it) so that the next row can be fetched while the current one is solved.
+struct VRow {
+    int ia, ib, cnt;
+    float mA, mB, iA, iB, friction, tspeed, tm0, tm1, nm0, nm1, b0, b1, K0, K1, K2, K3, N0, N1, N2, N3;
+    V2 n, rA0, rA1, rB0, rB1;
+    float ni0, ni1, ti0, ti1;
+};
+
+// A contact row's position-solver fields (b2ContactPositionConstraint), loaded in one batch.
+struct PRow {
+    int ia, ib, cnt, mtype;
+    V2 lcA, lcB, ln, lp, pl0, pl1;
+    float radA, radB, mA, mB, iA, iB;
+};
+
+// The position-solver fields of contact slot `slot` from its manifold and its bodies.
+GOI_D PRow prow_of(const DModel& m, const World& W, int slot) {
+    PRow p;
+    p.ia = W.ba(slot); p.ib = W.bb(slot);
+    p.cnt = W.ccount(slot); p.mtype = W.i32(GOI_C_MTYPE, slot);
+    p.lcA = W.v2(GOI_B_LOCAL_CENTER, p.ia); p.lcB = W.v2(GOI_B_LOCAL_CENTER, p.ib);
+    p.ln = W.v2(GOI_C_LOCAL_NORMAL, slot); p.lp = W.v2(GOI_C_LOCAL_POINT, slot);
+    p.pl0 = W.v2(GOI_C_POINT_LOCAL, 2 * slot); p.pl1 = W.v2(GOI_C_POINT_LOCAL, 2 * slot + 1);
+    p.radA = m.fix[W.fa(slot)].radius; p.radB = m.fix[W.fb(slot)].radius;
+    p.mA = W.f(GOI_B_INV_MASS, p.ia); p.mB = W.f(GOI_B_INV_MASS, p.ib);
+    p.iA = W.f(GOI_B_INV_INERTIA, p.ia); p.iB = W.f(GOI_B_INV_INERTIA, p.ib);
+    return p;
+}
+
+// b2ContactSolver constructor + InitializeVelocityConstraints for contact slot `slot` (contact_solver.py:32-147), whose
+// position-solver fields are p. Body positions/velocities from the LDS arrays; qA/qB the bodies' rotations.
+GOI_D VRow vrow_of(const World& W, const Bodies& bd, const PRow& p, int slot, bool warm, float dt_ratio, Rot qA, Rot qB,
+                   float velocity_threshold) {
+    VRow r;
+    const int ia = p.ia, ib = p.ib, mtype = p.mtype, cnt = p.cnt;
+    const float mA = p.mA, mB = p.mB, iA = p.iA, iB = p.iB, radA = p.radA, radB = p.radB;
+    r.ia = ia; r.ib = ib;
+    r.mA = mA; r.mB = mB; r.iA = iA; r.iB = iB;
+    r.ni0 = warm ? dt_ratio * W.f(GOI_C_NORMAL_IMPULSE, 2 * slot) : 0.0f;
+    r.ni1 = warm ? dt_ratio * W.f(GOI_C_NORMAL_IMPULSE, 2 * slot + 1) : 0.0f;
+    r.ti0 = warm ? dt_ratio * W.f(GOI_C_TANGENT_IMPULSE, 2 * slot) : 0.0f;
+    r.ti1 = warm ? dt_ratio * W.f(GOI_C_TANGENT_IMPULSE, 2 * slot + 1) : 0.0f;
+    r.friction = W.f(GOI_C_FRICTION, slot);
+    r.tspeed = W.f(GOI_C_TANGENT_SPEED, slot);
     const float restitution = W.f(GOI_C_RESTITUTION, slot);
     const V2 cA = bd.c(ia), cB = bd.c(ib);
     const V2 vA = bd.v(ia), vB = bd.v(ib);
     const float wA = bd.w(ia), wB = bd.w(ib);
     Xf xfA, xfB;
     xfA.q = qA; xfB.q = qB;
-    xfA.p = cA - mul(qA, lcA);
-    xfB.p = cB - mul(qB, lcB);
+    xfA.p = cA - mul(qA, p.lcA);
+    xfB.p = cB - mul(qB, p.lcB);
     // b2WorldManifold::Initialize
     V2 n = mk(1.0f, 0.0f), p0, p1;
     if (mtype == kCircles) {
-        const V2 pA = mul(xfA, lp), pB = mul(xfB, pl0);
+        const V2 pA = mul(xfA, p.lp), pB = mul(xfB, p.pl0);
         const V2 d = pB - pA;
         if (dot(d, d) > kEps * kEps) {
             n = d;
@@ -204,35 +222,35 @@ GOI_D void cs_prepare(const DModel& m, const World& W, const Bodies& bd, const R
         const Xf& x1 = fa ? xfA : xfB;
         const Xf& x2 = fa ? xfB : xfA;
         const float r1 = fa ? radA : radB, r2 = fa ? radB : radA;
-        n = mul(x1.q, ln);
-        const V2 pp = mul(x1, lp);
-        const V2 q0 = mul(x2, pl0), q1 = mul(x2, pl1);
+        n = mul(x1.q, p.ln);
+        const V2 pp = mul(x1, p.lp);
+        const V2 q0 = mul(x2, p.pl0), q1 = mul(x2, p.pl1);
         p0 = 0.5f * ((q0 + (r1 - dot(q0 - pp, n)) * n) + (q0 - r2 * n));
         p1 = 0.5f * ((q1 + (r1 - dot(q1 - pp, n)) * n) + (q1 - r2 * n));
         if (!fa) n = -n;
     }
-    R.set2(i, CF_NX, n);
+    r.n = n;
     const V2 t = cross(n, 1.0f);
     const V2 pts[2] = {p0, p1};
     float rnA2[2], rnB2[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         const V2 rA = pts[j] - cA, rB = pts[j] - cB;
-        R.set2(i, CF_RA0 + 2 * j, rA);
-        R.set2(i, CF_RB0 + 2 * j, rB);
+        (j == 0 ? r.rA0 : r.rA1) = rA;
+        (j == 0 ? r.rB0 : r.rB1) = rB;
         const float rnA = cross(rA, n), rnB = cross(rB, n);
         rnA2[j] = rnA;
         rnB2[j] = rnB;
         const float kn = ((mA + mB) + iA * rnA * rnA) + iB * rnB * rnB;
         const float rtA = cross(rA, t), rtB = cross(rB, t);
         const float kt = ((mA + mB) + iA * rtA * rtA) + iB * rtB * rtB;
-        R.setf(i, CF_NMASS0 + j, kn > 0.0f ? 1.0f / kn : 0.0f);
-        R.setf(i, CF_TMASS0 + j, kt > 0.0f ? 1.0f / kt : 0.0f);
+        (j == 0 ? r.nm0 : r.nm1) = kn > 0.0f ? 1.0f / kn : 0.0f;
+        (j == 0 ? r.tm0 : r.tm1) = kt > 0.0f ? 1.0f / kt : 0.0f;
         const float vrel = dot(n, rel_vel(vB, wB, rB, vA, wA, rA));
-        R.setf(i, CF_BIAS0 + j, vrel < -velocity_threshold ? -restitution * vrel : 0.0f);
+        (j == 0 ? r.b0 : r.b1) = vrel < -velocity_threshold ? -restitution * vrel : 0.0f;
     }
-    int vcount = cnt;
-    float K0 = 0.0f, K1 = 0.0f, K2 = 0.0f, K3 = 0.0f, N0 = 0.0f, N1 = 0.0f, N2 = 0.0f, N3 = 0.0f;
+    r.cnt = cnt;
+    r.K0 = r.K1 = r.K2 = r.K3 = r.N0 = r.N1 = r.N2 = r.N3 = 0.0f;
     if (cnt == 2) {
         const float k11 = ((mA + mB) + iA * rnA2[0] * rnA2[0]) + iB * rnB2[0] * rnB2[0];
         const float k22 = ((mA + mB) + iA * rnA2[1] * rnA2[1]) + iB * rnB2[1] * rnB2[1];
@@ -240,44 +258,39 @@ GOI_D void cs_prepare(const DModel& m, const World& W, const Bodies& bd, const R
         if (k11 * k11 < 1000.0f * (k11 * k22 - k12 * k12)) {
             float det = k11 * k22 - k12 * k12;
             if (det != 0.0f) det = 1.0f / det;
-            K0 = k11; K1 = k12; K2 = k12; K3 = k22;
-            N0 = det * k22; N1 = -det * k12; N2 = -det * k12; N3 = det * k11;
+            r.K0 = k11; r.K1 = k12; r.K2 = k12; r.K3 = k22;
+            r.N0 = det * k22; r.N1 = -det * k12; r.N2 = -det * k12; r.N3 = det * k11;
         } else {
-            vcount = 1;
+            r.cnt = 1;
         }
     }
-    R.seti(i, CF_COUNT, vcount);
-    R.setf(i, CF_K0, K0); R.setf(i, CF_K1, K1); R.setf(i, CF_K2, K2); R.setf(i, CF_K3, K3);
-    R.setf(i, CF_NM0, N0); R.setf(i, CF_NM1, N1); R.setf(i, CF_NM2, N2); R.setf(i, CF_NM3, N3);
+    return r;
 }
 
-template <class BD>
-GOI_D void cs_warm_start(const BD& bd, const Rows& R, int i) {
-    const int ia = R.geti(i, CF_IA), ib = R.geti(i, CF_IB), cnt = R.geti(i, CF_COUNT);
-    const float mA = R.getf(i, CF_MA), mB = R.getf(i, CF_MB), iA = R.getf(i, CF_IIA), iB = R.getf(i, CF_IIB);
-    const V2 n = R.get2(i, CF_NX), t = cross(n, 1.0f);
-    V2 vA = bd.v(ia), vB = bd.v(ib);
-    float wA = bd.w(ia), wB = bd.w(ib);
-    for (int j = 0; j < cnt; ++j) {
-        const V2 P = R.getf(i, CF_NI0 + j) * n + R.getf(i, CF_TI0 + j) * t;
-        wA = wA - iA * cross(R.get2(i, CF_RA0 + 2 * j), P);
-        vA = vA - mA * P;
-        wB = wB + iB * cross(R.get2(i, CF_RB0 + 2 * j), P);
-        vB = vB + mB * P;
-    }
-    bd.set_v(ia, vA, wA);
-    bd.set_v(ib, vB, wB);
+// a contact row's fields into row i of the row tile, for the passes that read the rows from there
+GOI_D void store_prow(const Rows& R, int i, int slot, const PRow& p) {
+    R.seti(i, CF_SLOT, slot); R.seti(i, CF_IA, p.ia); R.seti(i, CF_IB, p.ib);
+    R.seti(i, CF_PC_COUNT, p.cnt); R.seti(i, CF_MTYPE, p.mtype);
+    R.setf(i, CF_MA, p.mA); R.setf(i, CF_MB, p.mB); R.setf(i, CF_IIA, p.iA); R.setf(i, CF_IIB, p.iB);
+    R.set2(i, CF_LN, p.ln); R.set2(i, CF_LP, p.lp); R.set2(i, CF_PL0, p.pl0); R.set2(i, CF_PL1, p.pl1);
+    R.set2(i, CF_LCA, p.lcA); R.set2(i, CF_LCB, p.lcB); R.setf(i, CF_RADA, p.radA); R.setf(i, CF_RADB, p.radB);
 }
-
-// b2ContactSolver::SolveVelocityConstraints for row i (contact_solver.py:194-279)
-// A contact row's velocity-solver fields, loaded in one batch (every field, whether or not the row's point count
-// uses it) so that the next row can be fetched while the current one is solved.
-struct VRow {
-    int ia, ib, cnt;
-    float mA, mB, iA, iB, friction, tspeed, tm0, tm1, nm0, nm1, b0, b1, K0, K1, K2, K3, N0, N1, N2, N3;
-    V2 n, rA0, rA1, rB0, rB1;
-    float ni0, ni1, ti0, ti1;
-};
+GOI_D void store_vrow(const Rows& R, int i, const VRow& r) {
+    R.setf(i, CF_NI0, r.ni0); R.setf(i, CF_NI1, r.ni1); R.setf(i, CF_TI0, r.ti0); R.setf(i, CF_TI1, r.ti1);
+    R.setf(i, CF_FRICTION, r.friction); R.setf(i, CF_TSPEED, r.tspeed); R.set2(i, CF_NX, r.n);
+    R.set2(i, CF_RA0, r.rA0); R.set2(i, CF_RA1, r.rA1); R.set2(i, CF_RB0, r.rB0); R.set2(i, CF_RB1, r.rB1);
+    R.setf(i, CF_NMASS0, r.nm0); R.setf(i, CF_NMASS1, r.nm1); R.setf(i, CF_TMASS0, r.tm0); R.setf(i, CF_TMASS1, r.tm1);
+    R.setf(i, CF_BIAS0, r.b0); R.setf(i, CF_BIAS1, r.b1);
+    R.seti(i, CF_COUNT, r.cnt);
+    R.setf(i, CF_K0, r.K0); R.setf(i, CF_K1, r.K1); R.setf(i, CF_K2, r.K2); R.setf(i, CF_K3, r.K3);
+    R.setf(i, CF_NM0, r.N0); R.setf(i, CF_NM1, r.N1); R.setf(i, CF_NM2, r.N2); R.setf(i, CF_NM3, r.N3);
+}
+GOI_D void cs_prepare(const DModel& m, const World& W, const Bodies& bd, const Rows& R, int i, int slot, bool warm,
+                      float dt_ratio, Rot qA, Rot qB, float velocity_threshold) {
+    const PRow p = prow_of(m, W, slot);
+    store_prow(R, i, slot, p);
+    store_vrow(R, i, vrow_of(W, bd, p, slot, warm, dt_ratio, qA, qB, velocity_threshold));
+}
 
 GOI_D VRow load_vrow(const Rows& R, int i) {
     VRow r;
@@ -294,6 +307,27 @@ GOI_D VRow load_vrow(const Rows& R, int i) {
     return r;
 }
 
+// the warm start of one row (contact_solver.py:165-184)
+template <class BD>
+GOI_D void warm_vrow(const BD& bd, const VRow& r) {
+    const V2 n = r.n, t = cross(n, 1.0f);
+    const V2 vA0 = bd.v(r.ia), vB0 = bd.v(r.ib);
+    const float wA0 = bd.w(r.ia), wB0 = bd.w(r.ib);
+    V2 vA = vA0, vB = vB0;
+    float wA = wA0, wB = wB0;
+    const auto point = [&](float ni, float ti, V2 rA, V2 rB) {
+        const V2 P = ni * n + ti * t;
+        wA = wA - r.iA * cross(rA, P);
+        vA = vA - r.mA * P;
+        wB = wB + r.iB * cross(rB, P);
+        vB = vB + r.mB * P;
+    };
+    if (r.cnt > 0) point(r.ni0, r.ti0, r.rA0, r.rB0);
+    if (r.cnt > 1) point(r.ni1, r.ti1, r.rA1, r.rB1);
+    bd.set_v(r.ia, vA, wA, vA0, wA0);
+    bd.set_v(r.ib, vB, wB, vB0, wB0);
+}
+
 // b2ContactSolver::SolveVelocityConstraints for one row (contact_solver.py:194-290): tangent rows first, then the
 // normal row or the 2-point block solver's four cases. Updates the row's impulses in r and the bodies in LDS.
 template <class BD>
@@ -302,8 +336,10 @@ GOI_D void solve_vrow(const BD& bd, VRow& r) {
     const float mA = r.mA, mB = r.mB, iA = r.iA, iB = r.iB;
     const V2 rA0 = r.rA0, rA1 = r.rA1, rB0 = r.rB0, rB1 = r.rB1;
     float ni0 = r.ni0, ni1 = r.ni1, ti0 = r.ti0, ti1 = r.ti1;
-    V2 vA = bd.v(r.ia), vB = bd.v(r.ib);
-    float wA = bd.w(r.ia), wB = bd.w(r.ib);
+    const V2 vA0 = bd.v(r.ia), vB0 = bd.v(r.ib);
+    const float wA0 = bd.w(r.ia), wB0 = bd.w(r.ib);
+    V2 vA = vA0, vB = vB0;
+    float wA = wA0, wB = wB0;
     // tangent constraints first
     if (r.cnt > 0) {
         const float vt = dot(rel_vel(vB, wB, rB0, vA, wA, rA0), t) - r.tspeed;
@@ -374,8 +410,8 @@ GOI_D void solve_vrow(const BD& bd, VRow& r) {
         }
     }
     r.ni0 = ni0; r.ni1 = ni1; r.ti0 = ti0; r.ti1 = ti1;
-    bd.set_v(r.ia, vA, wA);
-    bd.set_v(r.ib, vB, wB);
+    bd.set_v(r.ia, vA, wA, vA0, wA0);
+    bd.set_v(r.ib, vB, wB, vB0, wB0);
 }
 
 // ---- TOI velocity passes with one moving body
@@ -527,8 +563,7 @@ GOI_D void store_vimpulses(const Rows& R, int i, const VRow& r) {
 
 // rows i0..n-1 once each, in order, each loaded in one batch while the row before it is solved; two rows a loop
 // iteration, so the two row buffers alternate without copies between them
-template <class BD>
-GOI_D void cs_solve_velocity_sweep(const BD& bd, const Rows& R, int i0, int n) {
+GOI_D void cs_solve_velocity_sweep(const Bodies& bd, const Rows& R, int i0, int n) {
     if (n <= i0) return;
     VRow a = load_vrow(R, i0), b;
     for (int i = i0; i < n; i += 2) {
@@ -541,13 +576,6 @@ GOI_D void cs_solve_velocity_sweep(const BD& bd, const Rows& R, int i0, int n) {
         store_vimpulses(R, i + 1, b);
     }
 }
-
-// A contact row's position-solver fields (b2ContactPositionConstraint), loaded in one batch.
-struct PRow {
-    int ia, ib, cnt, mtype;
-    V2 lcA, lcB, ln, lp, pl0, pl1;
-    float radA, radB, mA, mB, iA, iB;
-};
 
 GOI_D PRow load_prow(const Rows& R, int i) {
     PRow r;
@@ -567,8 +595,10 @@ GOI_D float solve_prow(const BD& bd, const PRow& r, float baumgarte, float mA, f
                        float linear_slop, float max_linear_correction, RotMemo& qa, RotMemo& qb) {
     const V2 lcA = r.lcA, lcB = r.lcB, ln = r.ln, lp = r.lp;
     const float radA = r.radA, radB = r.radB;
-    V2 cA = bd.c(r.ia), cB = bd.c(r.ib);
-    float aA = bd.a(r.ia), aB = bd.a(r.ib);
+    const V2 cA0 = bd.c(r.ia), cB0 = bd.c(r.ib);
+    const float aA0 = bd.a(r.ia), aB0 = bd.a(r.ib);
+    V2 cA = cA0, cB = cB0;
+    float aA = aA0, aB = aB0;
     float min_sep = 0.0f;
     for (int j = 0; j < r.cnt; ++j) {
         Xf xfA, xfB;
@@ -599,6 +629,7 @@ GOI_D float solve_prow(const BD& bd, const PRow& r, float baumgarte, float mA, f
         }
         const V2 rA = p - cA, rB = p - cB;
         min_sep = bmin(min_sep, sep);
+        bd.note_sep(sep);
         const float C = bclamp(baumgarte * (sep + linear_slop), -max_linear_correction, 0.0f);
         const float rnA = cross(rA, n), rnB = cross(rB, n);
         const float K = ((mA + mB) + iA * rnA * rnA) + iB * rnB * rnB;
@@ -607,8 +638,8 @@ GOI_D float solve_prow(const BD& bd, const PRow& r, float baumgarte, float mA, f
         cA = cA - mA * P; aA = aA - iA * cross(rA, P);
         cB = cB + mB * P; aB = aB + iB * cross(rB, P);
     }
-    bd.set_c(r.ia, cA, aA);
-    bd.set_c(r.ib, cB, aB);
+    bd.set_c(r.ia, cA, aA, cA0, aA0);
+    bd.set_c(r.ib, cB, aB, cB0, aB0);
     return min_sep;
 }
 

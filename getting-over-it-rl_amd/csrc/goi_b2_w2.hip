@@ -1,4 +1,5 @@
 // goi_b2_w2.hip - the step for any dimensions, 2 worlds per wave (b2_waves.hpp).
+#define GOI_LANE_ROWS 1  // contact rows a lane holds (b2_step.hpp)
 #include "b2_waves.hpp"
 
 namespace goi {
