@@ -4,6 +4,11 @@ A device State has the reference's field names and logical shapes (N, *inner) (g
 torch tensors whose storage is worlds-minor: leaf L with inner shape S is one contiguous (prod(S), pitch) buffer
 viewed as (N, *S) with stride 1 on the world axis. `state_view` hands those buffers to the C ABI without copies.
 """
+import array
+import ctypes
+import functools
+import operator
+
 import numpy as np
 import torch
 
@@ -28,22 +33,43 @@ def packed_words(dims):
     return words
 
 
+@functools.lru_cache(maxsize=64)
+def _spec(n, dims, pitch):
+    """What the leaves of n worlds of capacities dims with a pitch look like, in ABI order: dtypes, shapes, strides
+    (worlds-minor), and their byte offsets as the consecutive parts of one buffer, with that buffer's bytes."""
+    dtypes, shapes, strides = [], [], []
+    for _, _, dt, inner in wd.LEAVES:
+        shape = wd.leaf_shape(inner, dims)
+        want, acc = [], pitch
+        for d in reversed(shape):
+            want.insert(0, acc)
+            acc *= d
+        dtypes.append(_dtype(dt))
+        shapes.append((n,) + shape)
+        strides.append((1, *want))
+    offsets = [4 * w * pitch for w in packed_words(dims)]
+    return dtypes, shapes, strides, offsets[:-1], offsets[-1]
+
+
+def _carve(buf, n, dims, pitch):
+    """The State whose leaves are the consecutive parts of the byte buffer buf."""
+    dtypes, shapes, strides, offsets, _ = _spec(n, dims, pitch)
+    typed = {torch.float32: buf.view(torch.float32), torch.int32: buf.view(torch.int32), torch.bool: buf.view(torch.bool)}
+    size = {torch.float32: 4, torch.int32: 4, torch.bool: 1}
+    return wd.from_leaves([typed[dt].as_strided(sh, st, off // size[dt])
+                           for dt, sh, st, off in zip(dtypes, shapes, strides, offsets)])
+
+
 def empty_device_state(n, dims, device="cuda", pitch=None, packed=True):
-    """An uninitialised device State of n worlds with capacities dims = (B, R, J, C), pitch n by default. With a pitch
-    that is a multiple of 64 the leaves are by default the consecutive parts of one buffer (the packed layout), which
-    lets the step address every leaf from one base pointer; packed=False, or another pitch, gives one buffer per
-    leaf."""
+    """An uninitialised device State of n worlds with capacities dims = (B, R, J, C), pitch n by default. The leaves
+    are by default the consecutive parts of one buffer, which a clone copies whole; with a pitch that is a multiple of
+    64 that is the packed layout, which lets the step address every leaf from one base pointer. packed=False gives one
+    buffer per leaf."""
     pitch = n if pitch is None else pitch
+    dims = tuple(dims)
+    if packed and pitch > 0:
+        return _carve(torch.empty(_spec(n, dims, pitch)[4], dtype=torch.uint8, device=device), n, dims, pitch)
     vals = []
-    if packed and pitch > 0 and pitch % 64 == 0:
-        words = packed_words(dims)
-        buf = torch.empty(words[-1] * 4 * pitch, dtype=torch.uint8, device=device)
-        for (_, _, dt, inner), w in zip(wd.LEAVES, words):
-            shape = wd.leaf_shape(inner, dims)
-            nbytes = int(np.prod(shape, dtype=np.int64)) * np.dtype(dt).itemsize * pitch
-            part = buf[4 * w * pitch:4 * w * pitch + nbytes].view(_dtype(dt)).view(tuple(shape) + (pitch,))
-            vals.append(part[..., :n].movedim(-1, 0))
-        return wd.from_leaves(vals)
     for _, _, dt, inner in wd.LEAVES:
         shape = wd.leaf_shape(inner, dims)
         buf = torch.empty(tuple(shape) + (pitch,), dtype=_dtype(dt), device=device)
@@ -70,13 +96,41 @@ def to_host(state):
 
 def clone(state):
     """A deep copy of a device State in the same layout."""
+    return clone_view(state)[1]()
+
+
+def clone_view(state):
+    """A State's copy as (its GoiStateView, a function that returns the State): a caller that launches work on the copy
+    does so before the copy's 71 tensors are made. The view is None for a State that state_view would not take."""
     leaves = wd.leaves(state)
     n = leaves[0].shape[0]
     dims = wd.dims(state)
+    found = _match(state, leaves, n, dims)
+    buf = None if found is None else _copy_buffer(leaves, n, dims, *found)
+    if buf is not None:
+        pitch, base = found[0], buf.data_ptr()
+        return _view(n, dims, pitch, [base + o for o in _spec(n, dims, pitch)[3]]), lambda: _carve(buf, n, dims, pitch)
     out = empty_device_state(n, dims, leaves[0].device)
     for dst, src in zip(wd.leaves(out), leaves):
         dst.copy_(src)
-    return out
+    return None, lambda: out
+
+
+def _copy_buffer(leaves, n, dims, pitch, ptrs):
+    """A copy of the one buffer whose consecutive parts the (checked) leaves are, by a single device copy, or None where
+    the leaves are not laid out so."""
+    if pitch <= 0:
+        return None
+    _, _, _, offsets, nbytes = _spec(n, dims, pitch)
+    base = ptrs[0]
+    if ptrs != [base + o for o in offsets]:
+        return None
+    store = leaves[0].untyped_storage()
+    start = base - store.data_ptr()
+    if store.nbytes() - start < nbytes:
+        return None
+    src = torch.empty(0, dtype=torch.uint8, device=leaves[0].device).set_(store, start, (nbytes,))
+    return torch.empty_like(src).copy_(src)
 
 
 def pitch_of(state):
@@ -85,13 +139,32 @@ def pitch_of(state):
     return t.stride(-1) if t.dim() > 1 else t.shape[0]
 
 
-def state_view(state):
-    """GoiStateView over a device State; checks the worlds-minor layout."""
-    leaves = wd.leaves(state)
-    n = leaves[0].shape[0]
-    B, R, J, C = wd.dims(state)
-    v = GoiStateView()
-    v.n_worlds = n
+_SHAPE, _DTYPE, _DEVICE = (operator.attrgetter(a) for a in ("shape", "dtype", "device"))
+
+
+def _match(state, leaves, n, dims):
+    """(pitch, leaf addresses) of a GPU State in the worlds-minor layout, None for anything else. The leaves' types,
+    shapes, strides and devices are compared as whole lists."""
+    try:
+        pitch, device = state.bodies.xf_p.stride(-1), leaves[0].device
+        if device.type != "cuda" or pitch < n:
+            return None
+        dtypes, shapes, strides, _, _ = _spec(n, dims, pitch)
+        if (list(map(_DTYPE, leaves)) == dtypes and list(map(_SHAPE, leaves)) == shapes
+                and list(map(torch.Tensor.stride, leaves)) == strides
+                and list(map(_DEVICE, leaves)) == [device] * len(leaves)):
+            return pitch, list(map(torch.Tensor.data_ptr, leaves))
+    except (AttributeError, TypeError):  # not all tensors
+        pass
+    return None
+
+
+def _check(state, leaves, n, dims):
+    """_match, or what is wrong: the leaves walked one by one for the message."""
+    return _match(state, leaves, n, dims) or _check_leaves(leaves, n, dims)
+
+
+def _check_leaves(leaves, n, dims):
     pitch = None
     device = None
     for t, (_, name, dt, inner) in zip(leaves, wd.LEAVES):
@@ -102,7 +175,7 @@ def state_view(state):
         device = t.device
         if t.dtype != _dtype(dt):
             raise TypeError(f"leaf {name}: dtype {t.dtype}, expected {_dtype(dt)}")
-        shape = (n,) + wd.leaf_shape(inner, (B, R, J, C))
+        shape = (n,) + wd.leaf_shape(inner, dims)
         if tuple(t.shape) != shape:
             raise ValueError(f"leaf {name}: shape {tuple(t.shape)}, expected {shape}")
         if t.dim() > 1:
@@ -116,8 +189,23 @@ def state_view(state):
             pitch = p
         elif t.stride(0) != 1:
             raise ValueError(f"leaf {name}: world stride must be 1")
-    v.pitch = n if pitch is None else pitch
-    v.B, v.C, v.R, v.J = B, C, R, J
-    for i, t in enumerate(leaves):
-        v.leaf[i] = t.data_ptr()
+    return n if pitch is None else pitch, [t.data_ptr() for t in leaves]
+
+
+def _view(n, dims, pitch, ptrs):
+    v = GoiStateView()
+    v.n_worlds = n
+    v.pitch = pitch
+    v.B, v.R, v.J, v.C = dims
+    words = array.array("Q", ptrs)
+    ctypes.memmove(v.leaf, words.buffer_info()[0], 8 * len(ptrs))
     return v
+
+
+def state_view(state):
+    """GoiStateView over a device State; checks the worlds-minor layout."""
+    leaves = wd.leaves(state)
+    n = leaves[0].shape[0]
+    dims = wd.dims(state)
+    pitch, ptrs = _check(state, leaves, n, dims)
+    return _view(n, dims, pitch, ptrs)

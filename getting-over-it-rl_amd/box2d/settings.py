@@ -85,7 +85,7 @@ class Settings:
     def to_c(self):
         """The C ABI struct (include/goi_b2.h GoiSettings)."""
         from ._abi import GoiSettings
-        f = lambda n: float(F32(getattr(self, n)))  # noqa: E731
+        f = lambda n: getattr(self, n)  # noqa: E731  (a c_float field rounds as F32 does)
         return GoiSettings(
             velocity_iterations=int(self.velocity_iterations), position_iterations=int(self.position_iterations),
             linear_slop=f("linear_slop"), angular_slop=f("angular_slop"), polygon_radius=f("polygon_radius"),

@@ -97,19 +97,25 @@ def device_model(model, contact_capacity, device=None, state=None):
     return dm
 
 
-def step_(model, state, settings, dt, debug=None, stream=None):
-    """One step of every world of a device State, in place. Returns the same State."""
-    if getattr(settings, "solver", "hip") != "hip":
-        raise ValueError(f"Settings.solver={settings.solver!r}: this package steps on the GPU only ('hip')")
-    view = layout.state_view(state)
-    C = state.contacts.pair.shape[-1]
+def _launch(model, state, view, settings, dt, n, debug, stream):
+    """goi_step_n on a State's view; `state` is what a Model without body types or compact tables takes them from."""
     dev = state.contacts.pair.device
-    dm = device_model(model, C, dev, state)
+    dm = device_model(model, view.C, dev, state)
     cs = settings.to_c()
     st = torch.cuda.current_stream(dev).cuda_stream if stream is None else stream
     dbg = None if debug is None else ctypes.byref(debug)
-    _abi.check(dm.L.goi_step(dm.handle, ctypes.byref(view), ctypes.byref(cs), ctypes.c_float(np.float32(dt)),
-                             ctypes.c_void_p(st), dbg), dm.L)
+    _abi.check(dm.L.goi_step_n(dm.handle, ctypes.byref(view), ctypes.byref(cs), np.float32(dt), n, st, dbg), dm.L)
+
+
+def _need_hip(settings):
+    if getattr(settings, "solver", "hip") != "hip":
+        raise ValueError(f"Settings.solver={settings.solver!r}: this package steps on the GPU only ('hip')")
+
+
+def step_(model, state, settings, dt, debug=None, stream=None):
+    """One step of every world of a device State, in place. Returns the same State."""
+    _need_hip(settings)
+    _launch(model, state, layout.state_view(state), settings, dt, 1, debug, stream)
     return state
 
 
@@ -117,25 +123,20 @@ def step_n_(model, state, settings, dt, n, debug=None, stream=None):
     """n consecutive steps of every world of a device State in one launch, in place: the same State as n calls of
     step_ with the joint motor commands and forces left as they are (a caller's physics sub-steps per action).
     Returns the same State."""
-    if getattr(settings, "solver", "hip") != "hip":
-        raise ValueError(f"Settings.solver={settings.solver!r}: this package steps on the GPU only ('hip')")
-    view = layout.state_view(state)
-    C = state.contacts.pair.shape[-1]
-    dev = state.contacts.pair.device
-    dm = device_model(model, C, dev, state)
-    cs = settings.to_c()
-    st = torch.cuda.current_stream(dev).cuda_stream if stream is None else stream
-    dbg = None if debug is None else ctypes.byref(debug)
-    _abi.check(dm.L.goi_step_n(dm.handle, ctypes.byref(view), ctypes.byref(cs), ctypes.c_float(np.float32(dt)),
-                               ctypes.c_int32(int(n)), ctypes.c_void_p(st), dbg), dm.L)
+    _need_hip(settings)
+    _launch(model, state, layout.state_view(state), settings, dt, int(n), debug, stream)
     return state
 
 
 def step(model, state, settings, dt, axis_name=None):
     """b2World::Step (step.py:28-47) of a batched device State; returns a new State (the input is unchanged)."""
     del axis_name
-    out = layout.clone(state)
-    return step_(model, out, settings, dt)
+    _need_hip(settings)
+    view, made = layout.clone_view(state)
+    if view is None:
+        return step_(model, made(), settings, dt)
+    _launch(model, state, view, settings, dt, 1, None, None)
+    return made()
 
 
 def collide_(model, state, settings, stream=None):
@@ -158,7 +159,8 @@ def world_manifolds(model, state, stream=None):
     dev = state.contacts.pair.device
     dm = device_model(model, C, dev, state)
     pitch = view.pitch
-    bufs = [torch.zeros(shape + (pitch,), dtype=torch.float32, device=dev) for shape in ((C, 2), (C, 2, 2), (C, 2))]
+    # the kernel writes every word of the n worlds
+    bufs = [torch.empty(shape + (pitch,), dtype=torch.float32, device=dev) for shape in ((C, 2), (C, 2, 2), (C, 2))]
     st = torch.cuda.current_stream(dev).cuda_stream if stream is None else stream
     _abi.check(dm.L.goi_world_manifold(dm.handle, ctypes.byref(view), *[ctypes.c_void_p(b.data_ptr()) for b in bufs],
                                        ctypes.c_void_p(st)), dm.L)

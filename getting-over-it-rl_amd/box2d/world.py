@@ -202,7 +202,10 @@ def leaf_shape(inner, d):
 
 def leaves(state):
     """The 71 leaves of a State in ABI order."""
-    out = []
+    b, f, j, c, t = state.bodies, state.fixtures, state.joints, state.contacts, state.toi
+    if type(b) is Bodies and type(f) is Fixtures and type(j) is Joints and type(c) is Contacts and type(t) is ContactTOI:
+        return [*b, *f, *j, *c, state.gravity, state.inv_dt0, state.next_key, state.new_fixture, state.overflow, *t]
+    out = []  # another package's State classes, by name
     for group, name, _, _ in LEAVES:
         holder = state if group is None else getattr(state, group)
         out.append(getattr(holder, name))
@@ -211,16 +214,11 @@ def leaves(state):
 
 def from_leaves(vals):
     """A State from 71 leaves in ABI order."""
-    groups = {"bodies": [], "fixtures": [], "joints": [], "contacts": [], "toi": []}
-    scal = {}
-    for (group, name, _, _), v in zip(LEAVES, vals):
-        if group is None:
-            scal[name] = v
-        else:
-            groups[group].append(v)
-    return State(bodies=Bodies(*groups["bodies"]), fixtures=Fixtures(*groups["fixtures"]),
-                 joints=Joints(*groups["joints"]), contacts=Contacts(*groups["contacts"]), toi=ContactTOI(*groups["toi"]),
-                 **scal)
+    i = [0]
+    for part in (Bodies, Fixtures, Joints, Contacts):
+        i.append(i[-1] + len(part._fields))
+    return State(Bodies(*vals[:i[1]]), Fixtures(*vals[i[1]:i[2]]), Joints(*vals[i[2]:i[3]]), Contacts(*vals[i[3]:i[4]]),
+                 *vals[i[4]:i[4] + 5], ContactTOI(*vals[i[4] + 5:]))
 
 
 # ---------------------------------------------------------------- the host builder

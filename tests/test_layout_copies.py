@@ -1,0 +1,60 @@
+"""layout.clone and step() over every form of State they take: one buffer (any pitch), one buffer per leaf, a leaf that
+lies elsewhere, tensors in another order or on the CPU. The copy must hold the same words in memory of its own."""
+import numpy as np
+import pytest
+
+from util import b2, leaf_mismatches, wd
+
+torch = pytest.importorskip("torch")
+
+
+def _host_state(n):
+    return b2.scenes.make_config(1, n)
+
+
+def _copies(state, host):
+    out = b2.layout.clone(state)
+    assert leaf_mismatches(host, b2.layout.to_host(out)) == []
+    src = {t.untyped_storage().data_ptr() for t in wd.leaves(state)} - {0}  # 0: no worlds, no memory
+    assert not src & {t.untyped_storage().data_ptr() for t in wd.leaves(out)}
+    assert [tuple(t.shape) for t in wd.leaves(out)] == [tuple(t.shape) for t in wd.leaves(state)]
+    return out
+
+
+@pytest.mark.parametrize("n,pitch,packed", [(1, None, True), (3, None, True), (64, None, True), (50, 64, True),
+                                            (5, 9, False), (0, None, True)])
+def test_clone_on_the_cpu(n, pitch, packed):
+    _, _, st, _ = _host_state(max(n, 1))
+    if n == 0:
+        st = wd.from_leaves([x[:0] for x in wd.leaves(st)])
+    _copies(b2.layout.to_device(st, "cpu", pitch, packed), st)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", ["one", "odd", "pitch", "leaves", "elsewhere", "batch_major", "double"])
+def test_clone_and_step_on_the_gpu(oracle, case):
+    n = {"one": 1, "odd": 37, "pitch": 50}.get(case, 64)
+    s, m, st, cfg = _host_state(n)
+    dev = b2.layout.to_device(st, "cuda", 64 if case == "pitch" else None, case != "leaves")
+    if case == "elsewhere":  # one leaf replaced by a tensor of its own, in the same layout
+        key = dev.contacts.key
+        dev = dev._replace(contacts=dev.contacts._replace(key=torch.empty_strided(key.shape, key.stride(), dtype=key.dtype,
+                                                                                  device="cuda").copy_(key)))
+    elif case == "batch_major":  # state_view refuses it, a copy lays it out afresh
+        dev = wd.from_leaves([t.contiguous() for t in wd.leaves(dev)])
+        with pytest.raises(ValueError):
+            b2.layout.state_view(dev)
+    elif case == "double":
+        dev = dev._replace(bodies=dev.bodies._replace(w=dev.bodies.w.double()))
+        with pytest.raises(TypeError):
+            b2.layout.state_view(dev)
+    out = _copies(dev, st) if case != "double" else b2.layout.clone(dev)
+    if case == "pitch":
+        assert b2.layout.pitch_of(out) == 64
+    ref = oracle.step(m, st, s, cfg.dt)
+    stepped = b2.step(m, dev, s, cfg.dt)
+    assert leaf_mismatches(ref, b2.layout.to_host(stepped)) == []
+    b2.step_(m, out, s, cfg.dt)
+    assert leaf_mismatches(ref, b2.layout.to_host(out)) == []
+    if case != "double":
+        assert leaf_mismatches(st, b2.layout.to_host(dev)) == []  # the input as it was
