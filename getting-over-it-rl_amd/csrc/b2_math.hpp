@@ -311,6 +311,18 @@ GOI_D bool group_any(const Grp& g, bool p) {
     return x != 0;
 }
 
+// The group's lanes for which p holds, as a mask (bit i: lane i of the group), from one wavefront ballot.
+GOI_D unsigned long long group_ballot(const Group& g, bool p) {
+#ifdef GOI_HOST_BUILD
+    return p ? 1ull : 0ull;
+#else
+    const unsigned long long all = __ballot(p) >> ((int)threadIdx.x - g.s);
+    return g.g == 64 ? all : all & ((1ull << g.g) - 1ull);
+#endif
+}
+// Lane i of the group's v.
+GOI_D int group_lane(const Group& g, int v, int i) { return __shfl(v, (int)threadIdx.x - g.s + i, 64); }
+
 // b2Mat22::Solve / b2Mat33::Solve22
 GOI_D V2 solve22(float a11, float a12, float a21, float a22, V2 b) {
     float det = a11 * a22 - a12 * a21;

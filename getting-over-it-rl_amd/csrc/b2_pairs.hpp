@@ -207,26 +207,40 @@ GOI_D void collide_apply(const DModel& m, const World& W, const Rows& R) {
         const int e = min(q0 + 64, n);
         // 1. per list position (split over the lane group): the contact is destroyed (its fat boxes separated), and
         //    visiting it wakes its bodies (a destroyed contact that had points; an update that flips touching)
-        unsigned long long gone = 0ull, wakes = 0ull;
+        //    and whether a body of it that is not static is awake as the chunk begins
+        unsigned long long gone = 0ull, wakes = 0ull, visit = 0ull, asleep = 0ull, woken = 0ull;
         for (int i = q0 + W.sub; i < e; i += W.G) {
             const int k = W.order(i);
             const int t = W.cisl(k);
             const bool g = t < 0;
             const bool wk = g ? W.ccount(k) > 0 : (R.geti(t, MT_COUNT) > 0) != W.touching(k);
-            gone |= (unsigned long long)g << (i - q0);
-            wakes |= (unsigned long long)wk << (i - q0);
+            const unsigned long long pair = (1ull << W.ba(k)) | (1ull << W.bb(k)), bit = 1ull << (i - q0);
+            if (g) gone |= bit;
+            if (wk) wakes |= bit;
+            if (awake & pair & ~W.smask) {
+                visit |= bit;
+                if (wk) woken |= pair;
+            } else if (pair & ~W.smask) {
+                asleep |= bit;
+            }
         }
         gone = group_or(W.grp(), gone);
-        wakes = group_or(W.grp(), wakes);
-        // 2. Box2D's walk with its wake cascade, on bit masks: a contact is visited when one of its bodies is awake
-        //    and not static, and a visit that wakes makes both bodies awake for the rest of the walk
-        unsigned long long visit = 0ull;
-        for (int i = q0; i < e; ++i) {
-            const int k = W.order(i);
-            const unsigned long long pair = (1ull << W.ba(k)) | (1ull << W.bb(k));
-            if (!(awake & pair & ~W.smask)) continue;
-            visit |= 1ull << (i - q0);
-            if ((wakes >> (i - q0)) & 1ull) awake |= pair;
+        visit = group_or(W.grp(), visit);
+        if (!group_any(W.grp(), asleep != 0ull)) {
+            // every contact is visited whatever wakes on the way
+            awake |= group_or(W.grp(), woken);
+        } else {
+            // 2. Box2D's walk with its wake cascade, on bit masks: a contact is visited when one of its bodies is awake
+            //    and not static, and a visit that wakes makes both bodies awake for the rest of the walk
+            wakes = group_or(W.grp(), wakes);
+            visit = 0ull;
+            for (int i = q0; i < e; ++i) {
+                const int k = W.order(i);
+                const unsigned long long pair = (1ull << W.ba(k)) | (1ull << W.bb(k));
+                if (!(awake & pair & ~W.smask)) continue;
+                visit |= 1ull << (i - q0);
+                if ((wakes >> (i - q0)) & 1ull) awake |= pair;
+            }
         }
         // 3. the visited contacts' destructions and updates (each touches only its own slot), split over the group
         for (int i = q0 + W.sub; i < e; i += W.G) {
