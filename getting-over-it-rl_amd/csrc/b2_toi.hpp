@@ -84,29 +84,23 @@ GOI_D void restore(const World& W, int b, const SweepBackup& k) {
 
 // ---------------------------------------------------------------- distance proxies and GJK (toi.py:116-294)
 
-// b2DistanceProxy held in registers: the fixture's 8 vertex slots are loaded once, in one batch (the slots past
-// `count` are padding and never selected), so GJK's support searches and vertex lookups stay off memory.
+// b2DistanceProxy held in registers: the fixture's 8 vertex slots are loaded once, in one batch, so GJK's support
+// searches stay off memory. The slots past the count repeat vertex 0, which a search for the first largest dot never
+// selects over it, so the searches need no test against the count.
 struct Proxy {
     V2 v[kPoly];
     int count;
     float radius;
-    // vertex i (0 <= i < count) without dynamic register indexing: a chain of selects that starts from a constant
-    // (a chain of selects between loads would fold into one load from a selected address, which keeps the vertex
-    // array in private scratch memory)
-    GOI_D V2 at(int i) const {
-        V2 r = mk(0.0f, 0.0f);
-#pragma unroll
-        for (int j = 0; j < kPoly; ++j)
-            if (i == j) r = v[j];
-        return r;
-    }
 };
 GOI_D Proxy proxy_of(const DModel& m, int f) {
     Proxy p;
-#pragma unroll
-    for (int j = 0; j < kPoly; ++j) p.v[j] = m.poly[16 * f + j];
     p.count = m.fix[f].count;
     p.radius = m.fix[f].radius;
+#pragma unroll
+    for (int j = 0; j < kPoly; ++j) {
+        p.v[j] = m.poly[16 * f + j];
+        if (j > 0 && j >= p.count) p.v[j] = p.v[0];
+    }
     return p;
 }
 // b2DistanceProxy::GetSupport and GetVertex together: the first index of the largest dot and its vertex, selected in
@@ -115,30 +109,32 @@ struct Support {
     V2 v;
     int i;
 };
-template <int kN>
-GOI_D Support support_over(const Proxy& p, V2 d) {
-    Support s;
-    s.i = 0;
-    s.v = p.v[0];
-    float bv = dot(p.v[0], d);
+template <int kFrom, int kTo>
+GOI_D void support_over(const Proxy& p, V2 d, Support& s, float& bv) {
 #pragma unroll
-    for (int i = 1; i < kN; ++i) {
+    for (int i = kFrom; i < kTo; ++i) {
         const float v = dot(p.v[i], d);
-        if (i < p.count && v > bv) {
+        if (v > bv) {
             s.i = i;
             s.v = p.v[i];
             bv = v;
         }
     }
-    return s;
 }
 GOI_D Support support(const Proxy& p, V2 d) {
-    if (p.count <= 4) return support_over<4>(p, d);
-    return support_over<kPoly>(p, d);
+    Support s;
+    s.i = 0;
+    s.v = p.v[0];
+    float bv = dot(p.v[0], d);
+    support_over<1, 4>(p, d, s, bv);
+    if (p.count > 4) support_over<4, kPoly>(p, d, s, bv);
+    return s;
 }
 
+// A simplex vertex, with the proxies' own vertices beside their indices, so that neither GJK's next call nor the
+// separation function looks them up by index (a chain of 24 selects); the witness points follow from them when GJK ends.
 struct SVert {
-    V2 wA, wB, w;
+    V2 w, lA, lB;
     float a;
     int iA, iB;
 };
@@ -146,6 +142,7 @@ struct SimplexCache {
     float metric;
     int count;
     int iA[3], iB[3];
+    V2 lA[3], lB[3];
 };
 
 GOI_D float metric(const SVert* v, int count) {
@@ -157,52 +154,55 @@ GOI_D float metric(const SVert* v, int count) {
 GOI_D void set_vertex(SVert& v, const Xf& xA, int iA, V2 lA, const Xf& xB, int iB, V2 lB) {
     v.iA = iA;
     v.iB = iB;
-    v.wA = mul(xA, lA);
-    v.wB = mul(xB, lB);
-    v.w = v.wB - v.wA;
+    v.lA = lA;
+    v.lB = lB;
+    v.w = mul(xB, lB) - mul(xA, lA);
 }
-GOI_D void set_vertex(SVert& v, const Proxy& pA, const Xf& xA, int iA, const Proxy& pB, const Xf& xB, int iB) {
-    set_vertex(v, xA, iA, pA.at(iA), xB, iB, pB.at(iB));
-}
-
-GOI_D void simplex_solve2(SVert* v, int& count) {
-    const V2 w1 = v[0].w, w2 = v[1].w, e12 = w2 - w1;
-    const float d12_2 = -dot(w1, e12);
-    if (d12_2 <= 0.0f) { v[0].a = 1.0f; count = 1; return; }
-    const float d12_1 = dot(w2, e12);
-    if (d12_1 <= 0.0f) { v[1].a = 1.0f; count = 1; v[0] = v[1]; return; }
-    const float inv = 1.0f / (d12_1 + d12_2);
-    v[0].a = d12_1 * inv;
-    v[1].a = d12_2 * inv;
-    count = 2;
-}
-
-GOI_D void simplex_solve3(SVert* v, int& count) {
-    const V2 w1 = v[0].w, w2 = v[1].w, w3 = v[2].w;
-    const V2 e12 = w2 - w1, e13 = w3 - w1, e23 = w3 - w2;
+// b2Simplex::Solve2 and Solve3 (count 2 or 3): the region of the origin first, then one division and selects, so that
+// lanes in different regions share their instructions (as branches, the regions of a wave's lanes ran one after another).
+// The barycentric coordinates of the slots past the new count stay as Box2D leaves them.
+GOI_D void simplex_solve(SVert* v, int& count) {
+    enum { kV1, kV2, kV3, kE12, kE13, kE23, kFace };
+    const V2 w1 = v[0].w, w2 = v[1].w;
+    const V2 e12 = w2 - w1;
     const float d12_1 = dot(w2, e12), d12_2 = -dot(w1, e12);
-    const float d13_1 = dot(w3, e13), d13_2 = -dot(w1, e13);
-    const float d23_1 = dot(w3, e23), d23_2 = -dot(w2, e23);
-    const float n123 = cross(e12, e13);
-    const float d123_1 = n123 * cross(w2, w3), d123_2 = n123 * cross(w3, w1), d123_3 = n123 * cross(w1, w2);
-    if (d12_2 <= 0.0f && d13_2 <= 0.0f) { v[0].a = 1.0f; count = 1; return; }
-    if (d12_1 > 0.0f && d12_2 > 0.0f && d123_3 <= 0.0f) {
-        const float inv = 1.0f / (d12_1 + d12_2);
-        v[0].a = d12_1 * inv; v[1].a = d12_2 * inv; count = 2; return;
+    int region = d12_2 <= 0.0f ? kV1 : d12_1 <= 0.0f ? kV2 : kE12;
+    float p = d12_1, q = d12_2, r = 0.0f, den = d12_1 + d12_2;
+    if (count == 3) {
+        const V2 w3 = v[2].w;
+        const V2 e13 = w3 - w1, e23 = w3 - w2;
+        const float d13_1 = dot(w3, e13), d13_2 = -dot(w1, e13);
+        const float d23_1 = dot(w3, e23), d23_2 = -dot(w2, e23);
+        const float n123 = cross(e12, e13);
+        const float d123_1 = n123 * cross(w2, w3), d123_2 = n123 * cross(w3, w1), d123_3 = n123 * cross(w1, w2);
+        // the first that holds, in Box2D's order
+        region = kFace;
+        if ((int)(d23_1 > 0.0f) & (int)(d23_2 > 0.0f) & (int)(d123_1 <= 0.0f)) region = kE23;
+        if ((int)(d13_1 <= 0.0f) & (int)(d23_1 <= 0.0f)) region = kV3;
+        if ((int)(d12_1 <= 0.0f) & (int)(d23_2 <= 0.0f)) region = kV2;
+        if ((int)(d13_1 > 0.0f) & (int)(d13_2 > 0.0f) & (int)(d123_2 <= 0.0f)) region = kE13;
+        if ((int)(d12_1 > 0.0f) & (int)(d12_2 > 0.0f) & (int)(d123_3 <= 0.0f)) region = kE12;
+        if ((int)(d12_2 <= 0.0f) & (int)(d13_2 <= 0.0f)) region = kV1;
+        p = region == kE13 ? d13_1 : region == kE23 ? d23_1 : region == kFace ? d123_1 : p;
+        q = region == kE13 ? d13_2 : region == kE23 ? d23_2 : region == kFace ? d123_2 : q;
+        r = d123_3;
+        den = region == kFace ? (p + q) + r : p + q;
     }
-    if (d13_1 > 0.0f && d13_2 > 0.0f && d123_2 <= 0.0f) {
-        const float inv = 1.0f / (d13_1 + d13_2);
-        v[0].a = d13_1 * inv; v[2].a = d13_2 * inv; count = 2; v[1] = v[2]; return;
-    }
-    if (d12_1 <= 0.0f && d23_2 <= 0.0f) { v[1].a = 1.0f; count = 1; v[0] = v[1]; return; }
-    if (d13_1 <= 0.0f && d23_1 <= 0.0f) { v[2].a = 1.0f; count = 1; v[0] = v[2]; return; }
-    if (d23_1 > 0.0f && d23_2 > 0.0f && d123_1 <= 0.0f) {
-        const float inv = 1.0f / (d23_1 + d23_2);
-        v[1].a = d23_1 * inv; v[2].a = d23_2 * inv; count = 2; v[0] = v[2]; return;
-    }
-    const float inv = 1.0f / ((d123_1 + d123_2) + d123_3);
-    v[0].a = d123_1 * inv; v[1].a = d123_2 * inv; v[2].a = d123_3 * inv;
-    count = 3;
+    const float inv = 1.0f / den;
+    const bool edge = region >= kE12;
+    p = edge ? p * inv : 1.0f;
+    q = edge ? q * inv : 1.0f;
+    // slot 0 takes vertex 2 (kV2) or 3 (kV3, kE23), slot 1 vertex 3 (kE13)
+    const float a1 = v[1].a, a2 = v[2].a;
+    const bool from2 = region == kV2, from3 = (region == kV3) | (region == kE23), one3 = region == kE13;
+    const auto take = [&](SVert& x, const SVert& y) { x.w = y.w; x.lA = y.lA; x.lB = y.lB; x.iA = y.iA; x.iB = y.iB; };
+    if (from2) take(v[0], v[1]);
+    if (from3) take(v[0], v[2]);
+    if (one3) take(v[1], v[2]);
+    v[0].a = region == kE23 ? q : p;
+    v[1].a = region == kE23 ? p : (region == kV1) | (region == kV3) ? a1 : q;
+    v[2].a = region == kFace ? r * inv : (region == kV3) | (region == kE13) | (region == kE23) ? q : a2;
+    count = region < kE12 ? 1 : region == kFace ? 3 : 2;
 }
 
 // b2Distance (useRadii = false): the distance and the updated simplex cache. The simplex, the saved indices and
@@ -214,18 +214,18 @@ GOI_D float gjk_distance(SimplexCache& cache, const Proxy& pA, const Xf& xA, con
     for (int i = 0; i < 3; ++i) {
         v[i].a = 0.0f;
         v[i].iA = 0; v[i].iB = 0;
-        v[i].wA = mk(0.0f, 0.0f); v[i].wB = v[i].wA; v[i].w = v[i].wA;
+        v[i].w = v[i].lA = v[i].lB = mk(0.0f, 0.0f);
     }
     int count = cache.count;
 #pragma unroll
     for (int i = 0; i < 3; ++i)
-        if (i < count) set_vertex(v[i], pA, xA, cache.iA[i], pB, xB, cache.iB[i]);
+        if (i < count) set_vertex(v[i], xA, cache.iA[i], cache.lA[i], xB, cache.iB[i], cache.lB[i]);
     if (count > 1) {
         const float m1 = cache.metric, m2 = metric(v, count);
         if (m2 < 0.5f * m1 || 2.0f * m1 < m2 || m2 < kEps) count = 0;
     }
     if (count == 0) {
-        set_vertex(v[0], pA, xA, 0, pB, xB, 0);
+        set_vertex(v[0], xA, 0, pA.v[0], xB, 0, pB.v[0]);
         v[0].a = 1.0f;
         count = 1;
     }
@@ -235,8 +235,7 @@ GOI_D float gjk_distance(SimplexCache& cache, const Proxy& pA, const Xf& xA, con
 #pragma unroll
         for (int i = 0; i < 3; ++i)
             if (i < save) { saveA[i] = v[i].iA; saveB[i] = v[i].iB; }
-        if (count == 2) simplex_solve2(v, count);
-        else if (count == 3) simplex_solve3(v, count);
+        if (count > 1) simplex_solve(v, count);
         if (count == 3) break;
         V2 d;
         if (count == 1) {
@@ -261,22 +260,22 @@ GOI_D float gjk_distance(SimplexCache& cache, const Proxy& pA, const Xf& xA, con
         if (dup) break;
         ++count;
     }
-    V2 pa, pb;
-    if (count == 1) {
-        pa = v[0].wA;
-        pb = v[0].wB;
-    } else if (count == 2) {
-        pa = v[0].a * v[0].wA + v[1].a * v[1].wA;
-        pb = v[0].a * v[0].wB + v[1].a * v[1].wB;
-    } else {
-        pa = (v[0].a * v[0].wA + v[1].a * v[1].wA) + v[2].a * v[2].wA;
+    const V2 a0 = mul(xA, v[0].lA), b0 = mul(xB, v[0].lB);
+    V2 pa = a0, pb = b0;
+    if (count > 1) {
+        const V2 a1 = mul(xA, v[1].lA), b1 = mul(xB, v[1].lB);
+        pa = v[0].a * a0 + v[1].a * a1;
+        pb = v[0].a * b0 + v[1].a * b1;
+    }
+    if (count == 3) {
+        pa = pa + v[2].a * mul(xA, v[2].lA);
         pb = pa;
     }
     cache.metric = metric(v, count);
     cache.count = count;
 #pragma unroll
     for (int i = 0; i < 3; ++i)
-        if (i < count) { cache.iA[i] = v[i].iA; cache.iB[i] = v[i].iB; }
+        if (i < count) { cache.iA[i] = v[i].iA; cache.iB[i] = v[i].iB; cache.lA[i] = v[i].lA; cache.lB[i] = v[i].lB; }
     return length(pa - pb);
 }
 
@@ -288,64 +287,52 @@ struct SepFn {
     V2 axis, lp;
 };
 
-GOI_D SepFn sep_init(const SimplexCache& cache, const Proxy& pA, const Sweep& sA, const Proxy& pB, const Sweep& sB,
-                     float t1, RotMemo& ma, RotMemo& mb) {
-    const Xf xA = sweep_xf(sA, t1, ma), xB = sweep_xf(sB, t1, mb);
+// The separation function of the simplex GJK ended with; xA, xB: the sweeps' transforms at t1, where it ran. A face of
+// A and a face of B take the same instructions with the two sides exchanged (lanes of different types do not diverge).
+GOI_D SepFn sep_init(const SimplexCache& cache, const Xf& xA, const Xf& xB) {
     SepFn f;
+    const bool points = cache.count == 1;
+    const bool faceB = cache.iA[0] == cache.iA[1];
+    f.type = points ? kSepPoints : faceB ? kSepFaceB : kSepFaceA;
+    const V2 u1 = faceB ? cache.lB[0] : cache.lA[0], u2 = faceB ? cache.lB[1] : cache.lA[1];  // the face
+    const V2 a0 = mul(xA, cache.lA[0]), b0 = mul(xB, cache.lB[0]);
+    f.axis = points ? b0 - a0 : cross(u2 - u1, 1.0f);
+    normalize(f.axis);
     f.lp = mk(0.0f, 0.0f);
-    if (cache.count == 1) {
-        f.type = kSepPoints;
-        f.axis = mul(xB, pB.at(cache.iB[0])) - mul(xA, pA.at(cache.iA[0]));
-        normalize(f.axis);
-    } else if (cache.iA[0] == cache.iA[1]) {
-        f.type = kSepFaceB;
-        const V2 b1 = pB.at(cache.iB[0]), b2 = pB.at(cache.iB[1]);
-        f.axis = cross(b2 - b1, 1.0f);
-        normalize(f.axis);
-        const V2 n = mul(xB.q, f.axis);
-        f.lp = 0.5f * (b1 + b2);
-        if (dot(mul(xA, pA.at(cache.iA[0])) - mul(xB, f.lp), n) < 0.0f) f.axis = -f.axis;
-    } else {
-        f.type = kSepFaceA;
-        const V2 a1 = pA.at(cache.iA[0]), a2 = pA.at(cache.iA[1]);
-        f.axis = cross(a2 - a1, 1.0f);
-        normalize(f.axis);
-        const V2 n = mul(xA.q, f.axis);
-        f.lp = 0.5f * (a1 + a2);
-        if (dot(mul(xB, pB.at(cache.iB[0])) - mul(xA, f.lp), n) < 0.0f) f.axis = -f.axis;
+    if (!points) {
+        const Xf& own = faceB ? xB : xA;
+        const V2 n = mul(own.q, f.axis);
+        f.lp = 0.5f * (u1 + u2);
+        if (dot((faceB ? a0 : b0) - mul(own, f.lp), n) < 0.0f) f.axis = -f.axis;
     }
     return f;
 }
 
-// b2SeparationFunction::Evaluate at the support vertices lA = pA.at(iA), lB = pB.at(iB) that FindMinSeparation chose
-// (those of a face's own proxy unused), looked up once by the caller for all the root finder's steps
-GOI_D float sep_eval(const SepFn& f, const Sweep& sA, const Sweep& sB, V2 lA, V2 lB, float t, RotMemo& ma,
-                     RotMemo& mb) {
-    const Xf xA = sweep_xf(sA, t, ma), xB = sweep_xf(sB, t, mb);
-    if (f.type == kSepPoints) return dot(mul(xB, lB) - mul(xA, lA), f.axis);
-    if (f.type == kSepFaceA) return dot(mul(xB, lB) - mul(xA, f.lp), mul(xA.q, f.axis));
-    return dot(mul(xA, lA) - mul(xB, f.lp), mul(xB.q, f.axis));
+// b2SeparationFunction::Evaluate at the local points lA, lB that FindMinSeparation chose: the support vertices, and a
+// face's own point on its side
+GOI_D float sep_at(const SepFn& f, const Xf& xA, const Xf& xB, V2 n, V2 lA, V2 lB) {
+    const V2 pA = mul(xA, lA), pB = mul(xB, lB);
+    const bool faceB = f.type == kSepFaceB;
+    return dot((faceB ? pA : pB) - (faceB ? pB : pA), n);
+}
+GOI_D V2 sep_normal(const SepFn& f, const Xf& xA, const Xf& xB) {
+    const V2 n = mul(f.type == kSepFaceB ? xB.q : xA.q, f.axis);
+    return f.type == kSepPoints ? f.axis : n;
+}
+GOI_D float sep_eval(const SepFn& f, const Xf& xA, const Xf& xB, V2 lA, V2 lB) {
+    return sep_at(f, xA, xB, sep_normal(f, xA, xB), lA, lB);
 }
 
-// b2SeparationFunction::FindMinSeparation; lA, lB its support vertices (lA = (0, 0) for face A, lB for face B)
+// b2SeparationFunction::FindMinSeparation; lA, lB: its support vertices, the face's point on a face's own side
 GOI_D float sep_find_min(const SepFn& f, const Proxy& pA, const Sweep& sA, const Proxy& pB, const Sweep& sB, V2& lA,
                          V2& lB, float t, RotMemo& ma, RotMemo& mb) {
     const Xf xA = sweep_xf(sA, t, ma), xB = sweep_xf(sB, t, mb);
-    if (f.type == kSepPoints) {
-        lA = support(pA, mulT(xA.q, f.axis)).v;
-        lB = support(pB, mulT(xB.q, -f.axis)).v;
-        return dot(mul(xB, lB) - mul(xA, lA), f.axis);
-    }
-    if (f.type == kSepFaceA) {
-        const V2 n = mul(xA.q, f.axis);
-        lA = mk(0.0f, 0.0f);
-        lB = support(pB, mulT(xB.q, -n)).v;
-        return dot(mul(xB, lB) - mul(xA, f.lp), n);
-    }
-    const V2 n = mul(xB.q, f.axis);
-    lB = mk(0.0f, 0.0f);
-    lA = support(pA, mulT(xA.q, -n)).v;
-    return dot(mul(xA, lA) - mul(xB, f.lp), n);
+    const V2 n = sep_normal(f, xA, xB);
+    lA = support(pA, mulT(xA.q, f.type == kSepPoints ? n : -n)).v;
+    lB = support(pB, mulT(xB.q, -n)).v;
+    if (f.type == kSepFaceA) lA = f.lp;
+    if (f.type == kSepFaceB) lB = f.lp;
+    return sep_at(f, xA, xB, n, lA, lB);
 }
 
 enum { kToiUnknown = 0, kToiFailed = 1, kToiOverlapped = 2, kToiTouching = 3, kToiSeparated = 4 };
@@ -373,10 +360,11 @@ GOI_D int time_of_impact(const Proxy& pA, Sweep sA, const Proxy& pB, Sweep sB, f
     t_out = 1.0f;
     RotMemo ma, mb;
     for (int iter = 0;;) {
-        const float dist = gjk_distance(cache, pA, sweep_xf(sA, t1, ma), pB, sweep_xf(sB, t1, mb));
+        const Xf xA1 = sweep_xf(sA, t1, ma), xB1 = sweep_xf(sB, t1, mb);
+        const float dist = gjk_distance(cache, pA, xA1, pB, xB1);
         if (dist <= 0.0f) { state = kToiOverlapped; t_out = 0.0f; break; }
         if (dist < target + tol) { state = kToiTouching; t_out = t1; break; }
-        const SepFn f = sep_init(cache, pA, sA, pB, sB, t1, ma, mb);
+        const SepFn f = sep_init(cache, xA1, xB1);
         bool done = false;
         float t2 = 1.0f;
         for (int push = 0;;) {
@@ -384,14 +372,14 @@ GOI_D int time_of_impact(const Proxy& pA, Sweep sA, const Proxy& pB, Sweep sB, f
             float s2 = sep_find_min(f, pA, sA, pB, sB, lA, lB, t2, ma, mb);
             if (s2 > target + tol) { state = kToiSeparated; t_out = 1.0f; done = true; break; }
             if (s2 > target - tol) { t1 = t2; break; }
-            float s1 = sep_eval(f, sA, sB, lA, lB, t1, ma, mb);
+            float s1 = sep_eval(f, xA1, xB1, lA, lB);
             if (s1 < target - tol) { state = kToiFailed; t_out = t1; done = true; break; }
             if (s1 <= target + tol) { state = kToiTouching; t_out = t1; done = true; break; }
             float a1 = t1, a2 = t2;
             for (int rc = 0;;) {
                 const float t = (rc & 1) ? a1 + (target - s1) * (a2 - a1) / (s2 - s1) : 0.5f * (a1 + a2);
                 ++rc;
-                const float s = sep_eval(f, sA, sB, lA, lB, t, ma, mb);
+                const float s = sep_eval(f, sweep_xf(sA, t, ma), sweep_xf(sB, t, mb), lA, lB);
                 if (babs(s - target) < tol) { t2 = t; break; }
                 if (s > target) { a1 = t; s1 = s; }
                 else { a2 = t; s2 = s; }
