@@ -320,7 +320,7 @@ GOI_D bool slot_has_pair(const World& W, int p) {
 }
 
 // b2ContactManager::FindNewContacts (pairs.py:134-178) without scanning the candidate list: one walk of the static
-// BVH with the union of the world's non-static fat AABBs; at a leaf, each entry is tested against each row's box and
+// BVH with the union of the world's non-static fat AABBs; at a leaf, each entry is tested against the rows' boxes and
 // a hit maps to its candidate index through leaf_cand; the few non-static/non-static candidates are tested directly.
 // New pairs (overlapping, a dynamic body, both active, no contact yet) take the lowest free slots in ascending
 // candidate order with keys in that order, and enter the contact list at its head (newest first); a full table
@@ -350,10 +350,10 @@ GOI_D void find_new_contacts(const DModel& m, const World& W, unsigned long long
         bool has = false;
 #pragma unroll
         for (int j = 0; j < kHeld; ++j) has |= held[j] == p;
-        return group_any(W.grp(), has);
+        return group_ballot(W.grp(), has) != 0ull;
     };
     // the fat boxes of all rows into the workspace; the queried rows on active bodies and a box around them
-    unsigned long long rows = 0ull;
+    unsigned long long rows = 0ull, dynamic = 0ull;  // and the rows of dynamic bodies
     float4 U = make_float4(kMaxFloat, kMaxFloat, -kMaxFloat, -kMaxFloat);
     bool nan_query = false;
     const auto row_box = [&](int r) {
@@ -363,6 +363,7 @@ GOI_D void find_new_contacts(const DModel& m, const World& W, unsigned long long
         W.set_qbox(r, q);
         if (!((query_rows >> r) & 1ull) || !W.active(m.row[r].body)) return;
         rows |= 1ull << r;
+        if (m.row[r].dynamic) dynamic |= 1ull << r;
         U.x = fminf(U.x, q.x); U.y = fminf(U.y, q.y); U.z = fmaxf(U.z, q.z); U.w = fmaxf(U.w, q.w);
         nan_query |= q.x != q.x || q.y != q.y || q.z != q.z || q.w != q.w;
     };
@@ -371,6 +372,7 @@ GOI_D void find_new_contacts(const DModel& m, const World& W, unsigned long long
         // filters the tree walk, and each of its hits is tested against the rows' own boxes)
         for (int r = W.sub; r < m.R; r += W.G) row_box(r);
         rows = group_or(W.grp(), rows);
+        dynamic = group_or(W.grp(), dynamic);
         nan_query = group_or(W.grp(), nan_query ? 1ull : 0ull) != 0ull;
         for (int d = 1; d < W.G; d <<= 1) {
             U.x = fminf(U.x, lane_partner(U.x, d)); U.y = fminf(U.y, lane_partner(U.y, d));
@@ -383,105 +385,140 @@ GOI_D void find_new_contacts(const DModel& m, const World& W, unsigned long long
     // b2TestOverlap finds a box with a NaN coordinate overlapping every box, so such a row meets every static leaf:
     // a NaN union box then passes every node and leaf test below (and the row's own tests decide)
     if (nan_query) U = make_float4(kNaN, kNaN, kNaN, kNaN);
-    // the static tree, depth first: the lane group tests a node's 8 child boxes together against the union box; per
-    // level, the node and the mask of its overlapping children not yet visited (registers, selected by level). An
-    // unused child slot holds an empty box (lower > upper), which a NaN union box would pass: the hit needs a
-    // non-empty box too (the Model's static boxes are finite, checked at goi_model_create).
+    // The static tree, depth first over its inner nodes. The lane group tests a node's 8 child boxes together against the
+    // union box, then takes the entries of all its leaves that pass, 8 lanes a leaf; per level, the node's inner
+    // children not yet visited (registers, selected by level). An unused child slot holds an empty box (lower > upper),
+    // which a NaN union box would pass: the hit needs a non-empty box too (the Model's static boxes are finite, checked
+    // at goi_model_create). What bounds the walk is the latency of its serial steps, so a lane tests its entry against
+    // the queried rows, and the lanes' candidates load together. An entry at a time, on every lane, the search took 32
+    // us of a pile world's 242 (16 rows, 4 worlds a wave) and 12 of a rig world's 162.
     if (rows && m.n_wnodes > 0) {
+        const Group g = W.grp();
+        const int per = g.g < 8 ? g.g : 8;             // lanes a leaf
+        const int at_once = g.g < 8 ? 1 : g.g >> 3;    // leaves at once
+        const auto leaves = [&](int nd, unsigned children) {
+            for (unsigned left = children; left;) {
+                unsigned mine = left;
+                for (int i = 0; i < at_once; ++i) {
+                    if (i < (W.sub >> 3)) mine &= mine - 1u;
+                    left &= left - 1u;
+                }
+                const int ref = mine ? ~m.wnode[nd].ref[__builtin_ctz(mine)] : 0;
+                for (int j0 = 0; j0 < 8; j0 += per) {
+                    const int j = j0 + (W.sub & (per - 1)), at = (ref >> 4) + j;
+                    bool hit = j < (ref & 15);
+                    float4 fat = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                    unsigned long long with = rows;  // the rows whose pair with this entry may be new
+                    if (hit) {
+                        fat = m.leaf[at].fat;
+                        const int info = m.leaf[at].info;
+                        hit = overlap(fat, U) && W.active(info & 0xffff);
+                        if (!(info >> 16)) with &= dynamic;
+                    }
+                    if (group_ballot(g, hit) == 0ull) continue;
+                    unsigned long long found = 0ull;
+                    for (unsigned long long left = rows; left; left &= left - 1) {
+                        const int r = __builtin_ctzll(left);
+                        if (overlap(fat, W.get_qbox(r))) found |= 1ull << r;
+                    }
+                    found = hit ? found & with : 0ull;
+                    while (group_ballot(g, found != 0ull) != 0ull) {
+                        int p = -1;
+                        if (found) {
+                            p = m.leaf_cand[(size_t)at * m.R + __builtin_ctzll(found)];
+                            found &= found - 1;
+                        }
+                        for (unsigned long long left = group_ballot(g, p >= 0); left; left &= left - 1) {
+                            const int q = group_lane(g, p, __builtin_ctzll(left));
+                            if (!has_pair(q)) np.add(q);
+                        }
+                    }
+                }
+            }
+        };
+        // node nd's leaves that overlap are searched; returns the mask of its inner children that do
+        const auto visit = [&](int nd) {
+            unsigned hit = 0u, inner = 0u;
+            for (int j = W.sub; j < 8; j += g.g) {
+                const float4 b = m.wnode[nd].box[j];
+                if (overlap(U, b) && b.x <= b.z) hit |= 1u << j;
+                if (m.wnode[nd].ref[j] >= 0) inner |= 1u << j;
+            }
+            const unsigned both = (unsigned)group_or(g, (unsigned long long)(hit | inner << 8));
+            hit = both & 0xffu;
+            inner = both >> 8;
+            leaves(nd, hit & ~inner);
+            return hit & inner;
+        };
         int path[kWideDepth];
         unsigned masks[kWideDepth];
 #pragma unroll
         for (int l = 0; l < kWideDepth; ++l) { path[l] = 0; masks[l] = 0u; }
-        const auto children = [&](int nd) {
-            unsigned hit = 0u;
-            for (int j = W.sub; j < 8; j += W.G) {
-                const float4 b = m.wnode[nd].box[j];
-                if (overlap(U, b) && b.x <= b.z) hit |= 1u << j;
-            }
-            return group_or(W.grp(), hit);
-        };
-        masks[0] = children(0);
-        int level = 0;
+        int level = 0, next = 0;
         for (;;) {
-            int nd = 0;
-            unsigned cm = 0u;
+            const unsigned inner = visit(next);
 #pragma unroll
             for (int l = 0; l < kWideDepth; ++l)
-                if (l == level) { nd = path[l]; cm = masks[l]; }
-            if (cm == 0u) {
-                if (level == 0) break;
-                --level;
-                continue;
-            }
-            const int k = __builtin_ctz(cm);
+                if (l == level) { path[l] = next; masks[l] = inner; }
+            // the deepest level with an inner child left
+            int nd = 0;
+            unsigned cm = 0u;
+            level = -1;
+#pragma unroll
+            for (int l = 0; l < kWideDepth; ++l)
+                if (masks[l] != 0u) { level = l; nd = path[l]; cm = masks[l]; }
+            if (level < 0) break;
 #pragma unroll
             for (int l = 0; l < kWideDepth; ++l)
                 if (l == level) masks[l] = cm & (cm - 1u);
-            const int ref = m.wnode[nd].ref[k];
-            if (ref >= 0) {  // an inner node one level down
-                const unsigned hit = children(ref);
-                ++level;
-#pragma unroll
-                for (int l = 0; l < kWideDepth; ++l)
-                    if (l == level) { path[l] = ref; masks[l] = hit; }
-                continue;
-            }
-            // a leaf's entries (at most 8, one per lane) take the cheap union-box test; the few that pass are then
-            // tested row by row (one copy of that code, not one per entry), and only a hit reads its candidate index
-            const int first = (~ref) >> 4, cnt = (~ref) & 15;
-            unsigned hits = 0u;
-            for (int j = W.sub; j < cnt; j += W.G)
-                if (overlap(m.leaf[first + j].fat, U) && W.active(m.leaf[first + j].info & 0xffff)) hits |= 1u << j;
-            hits = group_or(W.grp(), hits);
-            for (; hits; hits &= hits - 1u) {
-                const int j = __builtin_ctz(hits);
-                const float4 fj = m.leaf[first + j].fat;
-                const int ij = m.leaf[first + j].info;
-                for (unsigned long long left = rows; left; left &= left - 1) {
-                    const int r = __builtin_ctzll(left);
-                    if (!overlap(fj, W.get_qbox(r))) continue;
-                    if (!(m.row[r].dynamic || (ij >> 16))) continue;
-                    const int p = m.leaf_cand[(size_t)(first + j) * m.R + r];
-                    if (p < 0 || has_pair(p)) continue;
-                    np.add(p);
-                }
-            }
+            next = m.wnode[nd].ref[__builtin_ctz(cm)];
+            ++level;
         }
     }
-    // non-static x non-static candidates
-    const auto dd_passes = [&](int i) {  // the tests that depend on candidate i alone
-        const int4 d = m.dd_info[i];     // candidate, rows, bodies
+    // non-static x non-static candidates, one a lane: the tests that depend on the candidate alone, then the ones that
+    // pass take the membership test and join the new pairs in order. A lane's next candidate loads during the tests, and
+    // one that passes comes from its lane's register: loaded again by every lane, a pile world's 25 or so took 11 us.
+    const int4 none = make_int4(0, 0, 0, 0);
+    int4 next = W.sub < m.n_dd ? m.dd_info[W.sub] : none;  // candidate, rows, bodies
+    for (int q0 = 0; q0 < m.n_dd; q0 += W.G) {
+        const int4 d = next;
+        const int i = q0 + W.sub;
+        if (i + W.G < m.n_dd) next = m.dd_info[i + W.G];
         const int ra = d.y & 0xff, rb = d.y >> 8, ba = d.z & 0xff, bb = d.z >> 8;
-        return (((query_rows >> ra) | (query_rows >> rb)) & 1ull) && overlap(W.get_qbox(ra), W.get_qbox(rb)) &&
-               (W.is_dynamic(ba) || W.is_dynamic(bb)) && W.active(ba) && W.active(bb);
-    };
-    if (m.R > 8) {
-        // many rows, so many candidates: those tests split over the group, 64 candidates at a time; the ones that
-        // pass then take the membership test and join the new pairs in order
-        for (int q0 = 0; q0 < m.n_dd; q0 += 64) {
-            const int e = min(q0 + 64, m.n_dd);
-            unsigned long long mk = 0ull;
-            for (int i = q0 + W.sub; i < e; i += W.G)
-                if (dd_passes(i)) mk |= 1ull << (i - q0);
-            for (unsigned long long left = group_or(W.grp(), mk); left; left &= left - 1) {
-                const int p = m.dd_info[q0 + __builtin_ctzll(left)].x;
-                if (!has_pair(p)) np.add(p);
-            }
+        const bool pass = i < m.n_dd && (((query_rows >> ra) | (query_rows >> rb)) & 1ull) &&
+                          overlap(W.get_qbox(ra), W.get_qbox(rb)) && (W.is_dynamic(ba) || W.is_dynamic(bb)) &&
+                          W.active(ba) && W.active(bb);
+        for (unsigned long long left = group_ballot(W.grp(), pass); left; left &= left - 1) {
+            const int p = group_lane(W.grp(), d.x, __builtin_ctzll(left));
+            if (!has_pair(p)) np.add(p);
         }
-    } else {
-        for (int i = 0; i < m.n_dd; ++i)
-            if (dd_passes(i) && !has_pair(m.dd_info[i].x)) np.add(m.dd_info[i].x);
     }
     if (np.total == 0) return;
     const int base_key = W.i32(GOI_S_NEXT_KEY, 0);
-    // the new contacts (keys base_key .. base_key + kept - 1) go to the head of the list, newest first
+    // The new contacts (keys base_key .. base_key + kept - 1) go to the head of the list, newest first. The list moves
+    // up a group's width at a time from its end, new contact i takes the i-th free slot, and the lanes create one each
+    // (every contact has a slot of its own; two that wake one body write the same words).
     const int nl = W.nlive();
-    for (int i = nl - 1; i >= 0; --i) W.order(i + np.kept) = W.order(i);
+    group_sync();
+    for (int e = nl; e > 0; e -= W.G) {
+        const int i = e - 1 - W.sub;
+        const int k = i >= 0 ? W.order(i) : 0;
+        group_sync();
+        if (i >= 0) W.order(i + np.kept) = k;
+        group_sync();
+    }
     W.nlive() = nl + np.kept;
-    int k = 0;
-    for (int i = 0; i < np.kept; ++i) {
-        while (W.pair(k) >= 0) ++k;
-        W.order(np.kept - 1 - i) = k;
+    for (int k0 = 0, n = 0; k0 < W.C && n < np.kept; k0 += W.G) {
+        const int k = k0 + W.sub;
+        const bool free = k < W.C && W.pair(k) < 0;
+        const unsigned long long mk = group_ballot(W.grp(), free);
+        const int i = n + __popcll(mk & ((1ull << W.sub) - 1ull));
+        if (free && i < np.kept) W.order(np.kept - 1 - i) = k;
+        n += __popcll(mk);
+    }
+    group_sync();
+    for (int i = W.sub; i < np.kept; i += W.G) {
+        const int k = W.order(np.kept - 1 - i);
         const int p = W.newp(i);
         const int2 ab = m.pair[p];
         const int a = ab.x, b = ab.y;
@@ -505,8 +542,8 @@ GOI_D void find_new_contacts(const DModel& m, const World& W, unsigned long long
         W.set_bodies(k, ba, bb);
         W.wake(ba);
         W.wake(bb);
-        ++k;
     }
+    group_sync();
     W.i32(GOI_S_NEXT_KEY, 0) = base_key + np.total;
     W.i32(GOI_S_OVERFLOW, 0) += np.total - np.kept;
 }

@@ -79,3 +79,29 @@ def test_solver_rows_beyond_the_lanes(oracle, monkeypatch, wpw, case):
     elif case == "nan":
         st.bodies.v[1::7, 9, 1] = np.nan
     _compare(m, st, s, cfg.dt, 6, oracle, nan_equal=True)
+
+
+@pytest.mark.parametrize("scene,slots,wpw", [(5, 128, 1), (5, 128, 2), (5, 128, 4), (5, 128, 8), (5, 20, 1), (5, 20, 8),
+                                             (4, 40, 16), (4, 40, 32), (4, 3, 32), (4, 3, 4)])
+def test_search_on_lane_groups(oracle, monkeypatch, scene, slots, wpw):
+    """FindNewContacts on lane groups of 64 down to 2: several leaves of the static tree at once or a leaf in parts, more
+    rows and non-static candidates than lanes and fewer, a first search that fills an empty contact list, later ones of
+    every pair beside the contacts that exist, a full table (pairs dropped), a row whose fat box is NaN (it meets every
+    leaf) and an inactive body."""
+    monkeypatch.setenv("GOI_WORLDS_PER_WAVE", str(wpw))
+    s, m, st, cfg = b2.scenes.make_config(scene, 37, capacity=slots)
+    dev, ref = b2.layout.to_device(st, "cuda"), oracle.copy(st)
+    for k in range(6):
+        if k in (2, 4):
+            ref = b2.layout.to_host(dev)
+            ref.new_fixture[:] = 1
+            if k == 4:
+                ref.bodies.active[::5, 2] = 0
+                ref.fixtures.fat[3::11, -1, 1] = np.nan
+            dev = b2.layout.to_device(ref, "cuda")
+        b2.step_(m, dev, s, cfg.dt)
+        oracle.step_(m, ref, s, cfg.dt)
+        bad = leaf_mismatches(ref, b2.layout.to_host(dev), True)
+        assert bad == [], f"step {k + 1}: {bad[:4]}"
+    live = (np.asarray(ref.contacts.pair) >= 0).sum(1)
+    assert live.max() == slots if slots in (3, 20) else live.max() > 4
