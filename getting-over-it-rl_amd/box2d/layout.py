@@ -52,12 +52,14 @@ def _spec(n, dims, pitch):
 
 
 def _carve(buf, n, dims, pitch):
-    """The State whose leaves are the consecutive parts of the byte buffer buf."""
+    """The State whose leaves are the consecutive parts of the byte buffer buf. Each float leaf is a tensor of its own to
+    autograd (.data): as views of one float tensor, a write that requires grad into one would make the next write into
+    any other an error."""
     dtypes, shapes, strides, offsets, _ = _spec(n, dims, pitch)
     typed = {torch.float32: buf.view(torch.float32), torch.int32: buf.view(torch.int32), torch.bool: buf.view(torch.bool)}
     size = {torch.float32: 4, torch.int32: 4, torch.bool: 1}
-    return wd.from_leaves([typed[dt].as_strided(sh, st, off // size[dt])
-                           for dt, sh, st, off in zip(dtypes, shapes, strides, offsets)])
+    parts = [typed[dt].as_strided(sh, st, off // size[dt]) for dt, sh, st, off in zip(dtypes, shapes, strides, offsets)]
+    return wd.from_leaves([t.data if dt is torch.float32 else t for dt, t in zip(dtypes, parts)])
 
 
 def empty_device_state(n, dims, device="cuda", pitch=None, packed=True):
@@ -105,7 +107,8 @@ def clone_view(state):
     leaves = wd.leaves(state)
     n = leaves[0].shape[0]
     dims = wd.dims(state)
-    found = _match(state, leaves, n, dims)
+    # a leaf that requires grad is copied leaf by leaf, so that its copy has it as its gradient's source
+    found = None if any(map(_REQUIRES_GRAD, leaves)) else _match(state, leaves, n, dims)
     buf = None if found is None else _copy_buffer(leaves, n, dims, *found)
     if buf is not None:
         pitch, base = found[0], buf.data_ptr()
@@ -139,7 +142,7 @@ def pitch_of(state):
     return t.stride(-1) if t.dim() > 1 else t.shape[0]
 
 
-_SHAPE, _DTYPE, _DEVICE = (operator.attrgetter(a) for a in ("shape", "dtype", "device"))
+_SHAPE, _DTYPE, _DEVICE, _REQUIRES_GRAD = map(operator.attrgetter, ("shape", "dtype", "device", "requires_grad"))
 
 
 def _match(state, leaves, n, dims):
@@ -154,7 +157,7 @@ def _match(state, leaves, n, dims):
                 and list(map(torch.Tensor.stride, leaves)) == strides
                 and list(map(_DEVICE, leaves)) == [device] * len(leaves)):
             return pitch, list(map(torch.Tensor.data_ptr, leaves))
-    except (AttributeError, TypeError):  # not all tensors
+    except (AttributeError, TypeError, RuntimeError):  # not all tensors, or tensors without memory
         pass
     return None
 

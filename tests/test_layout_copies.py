@@ -30,6 +30,31 @@ def test_clone_on_the_cpu(n, pitch, packed):
     _copies(b2.layout.to_device(st, "cpu", pitch, packed), st)
 
 
+def _grad_flows(device, n):
+    """A leaf that requires grad is the source of its copy's gradient, and the leaves are separate to autograd."""
+    _, _, st, _ = _host_state(n)
+    dev = b2.layout.to_device(st, device)
+    x = torch.ones_like(dev.bodies.v).requires_grad_()
+    dev.bodies.v.copy_(x)
+    dev.bodies.w.zero_()
+    assert dev.bodies.v.requires_grad and not dev.bodies.w.requires_grad
+    out = b2.layout.clone(dev)
+    assert not out.bodies.w.requires_grad
+    (g,) = torch.autograd.grad(out.bodies.v.sum(), x)
+    assert bool((g == 1).all())
+
+
+@pytest.mark.parametrize("n", [3, 64])
+def test_clone_keeps_autograd(n):
+    _grad_flows("cpu", n)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [3, 64])
+def test_clone_keeps_autograd_on_the_gpu(n):
+    _grad_flows("cuda", n)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("case", ["one", "odd", "pitch", "leaves", "elsewhere", "batch_major", "double"])
 def test_clone_and_step_on_the_gpu(oracle, case):
