@@ -146,63 +146,71 @@ __global__ void k_world_manifold(DModel m, Launch L, float* normal, float* point
 // (the State's toi.events: 8 or more, 3 or more, the rest). Each XCD keeps the contiguous range of groups xcd_group
 // gives it (block b runs on XCD b % 8): within the range, chunks of groups that share the State's 128-byte lines
 // (32 worlds) are ordered by class, each class in chunk order, so that a line's worlds stay in one XCD's L2. One
-// wavefront: per XCD, lane i takes a run of consecutive chunks, and the lanes' class sizes are scanned across the
-// wavefront. The step's results do not depend on the order.
+// wavefront per XCD's range (block x): lane i takes a run of consecutive chunks, and the lanes' class sizes are scanned
+// across the wavefront. The step's results do not depend on the order.
+//
+// It runs before the step with the GPU otherwise idle, and what bounds it is the latency of its loads: so the ranges run
+// side by side (one wavefront took them one after another), loads go 8 at a time, and a lane keeps its first 16 chunks'
+// classes instead of finding them twice. 65,536 pile worlds (16,384 groups): 160 -> 21 us, of a launch of 2.7 ms.
 __global__ void __launch_bounds__(kBlock) k_group_order(const int* events, const int* cost, int n, int wpw, int groups,
                                                         int* order) {
     constexpr int kClasses = 8;
     const int lane = threadIdx.x, lanes = blockDim.x;
     int top = 0;  // the longest block time of the previous launch
+#pragma unroll 8
     for (int g = lane; g < groups; g += lanes) top = max(top, cost[g]);
     for (int d = 1; d < lanes; d <<= 1) top = max(top, __shfl_xor(top, d, 64));
     const int cg = wpw < 32 ? 32 / wpw : 1;  // groups per chunk
     const int q = groups >> 3, r = groups & 7;
-    for (int x = 0; x < 8; ++x) {
-        const int base = x * q + min(x, r), size = q + (x < r ? 1 : 0);  // XCD x's groups
-        const int chunks = (size + cg - 1) / cg;
-        const int per = (chunks + lanes - 1) / lanes;
-        const int k0 = min(lane * per, chunks), k1 = min(k0 + per, chunks);
-        const auto span = [&](int k) { return min(cg, size - k * cg); };  // groups in chunk k
-        const auto cls = [&](int k) {
-            const int g0 = base + k * cg, g1 = g0 + span(k);
-            if (top > 0) {
-                int t = 0;
-                for (int g = g0; g < g1; ++g) t = max(t, cost[g]);
-                return t > 0 ? min(kClasses - 1, (int)(2.0f * log2f((float)top / (float)t))) : kClasses - 1;
-            }
-            int mx = 0;
-            for (int w = g0 * wpw; w < min(n, g1 * wpw); ++w) mx = max(mx, events[w]);
-            return mx >= 8 ? 0 : mx >= 3 ? 1 : 2;
-        };
-        int cnt[kClasses];  // this lane's groups per class
-#pragma unroll
-        for (int c = 0; c < kClasses; ++c) cnt[c] = 0;
-        for (int k = k0; k < k1; ++k) {
-            const int c = cls(k), g = span(k);
-#pragma unroll
-            for (int e = 0; e < kClasses; ++e) cnt[e] += e == c ? g : 0;
+    const int x = blockIdx.x;
+    const int base = x * q + min(x, r), size = q + (x < r ? 1 : 0);  // XCD x's groups
+    const int chunks = (size + cg - 1) / cg;
+    const int per = (chunks + lanes - 1) / lanes;
+    const int k0 = min(lane * per, chunks), k1 = min(k0 + per, chunks);
+    const auto span = [&](int k) { return min(cg, size - k * cg); };  // groups in chunk k
+    const auto cls = [&](int k) {
+        const int g0 = base + k * cg, g1 = g0 + span(k);
+        if (top > 0) {
+            int t = 0;
+#pragma unroll 8
+            for (int g = g0; g < g1; ++g) t = max(t, cost[g]);
+            return t > 0 ? min(kClasses - 1, (int)(2.0f * log2f((float)top / (float)t))) : kClasses - 1;
         }
-        int pos[kClasses];  // this lane's first position in each class
-        int before = 0;     // the groups of the classes before
+        int mx = 0;
+#pragma unroll 8
+        for (int w = g0 * wpw; w < min(n, g1 * wpw); ++w) mx = max(mx, events[w]);
+        return mx >= 8 ? 0 : mx >= 3 ? 1 : 2;
+    };
+    unsigned long long kept = 0ull;  // the classes of this lane's first 16 chunks, 4 bits each
+    int cnt[kClasses];               // this lane's groups per class
 #pragma unroll
-        for (int c = 0; c < kClasses; ++c) {
-            int incl = cnt[c];
-            for (int d = 1; d < lanes; d <<= 1) {
-                const int v = __shfl_up(incl, d, 64);
-                if (lane >= d) incl += v;
-            }
-            pos[c] = before + incl - cnt[c];
-            before += __shfl(incl, lanes - 1, 64);
+    for (int c = 0; c < kClasses; ++c) cnt[c] = 0;
+    for (int k = k0; k < k1; ++k) {
+        const int c = cls(k), g = span(k), j = k - k0;
+        if (j < 16) kept |= (unsigned long long)c << (4 * j);
+#pragma unroll
+        for (int e = 0; e < kClasses; ++e) cnt[e] += e == c ? g : 0;
+    }
+    int pos[kClasses];  // this lane's first position in each class
+    int before = 0;     // the groups of the classes before
+#pragma unroll
+    for (int c = 0; c < kClasses; ++c) {
+        int incl = cnt[c];
+        for (int d = 1; d < lanes; d <<= 1) {
+            const int v = __shfl_up(incl, d, 64);
+            if (lane >= d) incl += v;
         }
-        for (int k = k0; k < k1; ++k) {
-            const int c = cls(k), g = span(k);
-            int p = 0;
+        pos[c] = before + incl - cnt[c];
+        before += __shfl(incl, lanes - 1, 64);
+    }
+    for (int k = k0; k < k1; ++k) {
+        const int j = k - k0, c = j < 16 ? (int)(kept >> (4 * j)) & 15 : cls(k), g = span(k);
+        int p = 0;
 #pragma unroll
-            for (int e = 0; e < kClasses; ++e) p = e == c ? pos[e] : p;
-            for (int i = 0; i < g; ++i) order[8 * (p + i) + x] = base + k * cg + i;  // XCD x's (p + i)-th block
+        for (int e = 0; e < kClasses; ++e) p = e == c ? pos[e] : p;
+        for (int i = 0; i < g; ++i) order[8 * (p + i) + x] = base + k * cg + i;  // XCD x's (p + i)-th block
 #pragma unroll
-            for (int e = 0; e < kClasses; ++e) pos[e] += e == c ? g : 0;
-        }
+        for (int e = 0; e < kClasses; ++e) pos[e] += e == c ? g : 0;
     }
 }
 
@@ -818,7 +826,7 @@ static int launch_step(const GoiModel* M, const GoiStateView* state, const GoiSe
     const long resident = (long)cu_count() * blocks_per_cu(lds);
     if (order_buf && settings->continuous_physics && grid > resident) {
         int* cost = order_buf + state->pitch + 64;
-        hipLaunchKernelGGL(k_group_order, dim3(1), dim3(kBlock), 0, st,
+        hipLaunchKernelGGL(k_group_order, dim3(8), dim3(kBlock), 0, st,
                            static_cast<const int*>(state->leaf[GOI_T_EVENTS]), cost, state->n_worlds, L.wpw, grid,
                            order_buf);
         HIP_TRY(hipGetLastError());
