@@ -122,6 +122,18 @@ def test_config4_sanitized(host_step, tmp_path, packed, edges):
     assert all(("k_step_fixed" in ln) == packed for ln in launches), launches[:2]
 
 
+@pytest.mark.parametrize("n", [4093, 4500])
+def test_block_order_many_chunks(host_step, tmp_path, n):
+    """k_group_order with as many chunks a lane as it keeps classes of (16: 4,093 worlds in blocks of one, 512 or 511 to
+    an XCD, 32 to a chunk) and more (18), on event counts and then on block times; a block left out or run twice shows."""
+    m, st, s, dt, acts = config_case(4, n, 2)
+    p = tmp_path / "scn.bin"
+    write_scenario(p, m, st, s, dt, 2, True, acts)
+    r = run(host_step, p, "step")
+    check(r)
+    assert "k_group_order" in r.stderr
+
+
 @pytest.mark.parametrize("poison", ["8", "-1", "0"])
 def test_poisoned_scratch_sanitized(host_step, tmp_path, poison):
     """The benchmark rig (packed: the fixed instance) and the general kernel with the LDS workspaces and rows filled
