@@ -11,6 +11,7 @@ import operator
 
 import numpy as np
 import torch
+from torch.autograd import forward_ad
 
 from . import world as wd
 from ._abi import GoiStateView
@@ -107,16 +108,22 @@ def clone_view(state):
     leaves = wd.leaves(state)
     n = leaves[0].shape[0]
     dims = wd.dims(state)
-    # a leaf that requires grad is copied leaf by leaf, so that its copy has it as its gradient's source
-    found = None if any(map(_REQUIRES_GRAD, leaves)) else _match(state, leaves, n, dims)
+    found = _match(state, leaves, n, dims) if _memory_is_all(leaves) else None
     buf = None if found is None else _copy_buffer(leaves, n, dims, *found)
     if buf is not None:
         pitch, base = found[0], buf.data_ptr()
-        return _view(n, dims, pitch, [base + o for o in _spec(n, dims, pitch)[3]]), lambda: _carve(buf, n, dims, pitch)
+        view = _view(n, dims, pitch, [base + o for o in _spec(n, dims, pitch)[3]]) if buf.is_cuda else None
+        return view, lambda: _carve(buf, n, dims, pitch)
     out = empty_device_state(n, dims, leaves[0].device)
     for dst, src in zip(wd.leaves(out), leaves):
         dst.copy_(src)
     return None, lambda: out
+
+
+def _memory_is_all(leaves):
+    """Whether a copy of the leaves' memory copies all they are. A leaf that requires grad is copied as a leaf, so that its
+    copy has it as its gradient's source, and so is every leaf inside a forward-mode level, where it may have a tangent."""
+    return forward_ad._current_level < 0 and not any(map(_REQUIRES_GRAD, leaves))
 
 
 def _copy_buffer(leaves, n, dims, pitch, ptrs):
@@ -146,11 +153,11 @@ _SHAPE, _DTYPE, _DEVICE, _REQUIRES_GRAD = map(operator.attrgetter, ("shape", "dt
 
 
 def _match(state, leaves, n, dims):
-    """(pitch, leaf addresses) of a GPU State in the worlds-minor layout, None for anything else. The leaves' types,
-    shapes, strides and devices are compared as whole lists."""
+    """(pitch, leaf addresses) of a State in the worlds-minor layout on one device, None for anything else. The leaves'
+    types, shapes, strides and devices are compared as whole lists."""
     try:
         pitch, device = state.bodies.xf_p.stride(-1), leaves[0].device
-        if device.type != "cuda" or pitch < n:
+        if pitch < n:
             return None
         dtypes, shapes, strides, _, _ = _spec(n, dims, pitch)
         if (list(map(_DTYPE, leaves)) == dtypes and list(map(_SHAPE, leaves)) == shapes
@@ -163,8 +170,9 @@ def _match(state, leaves, n, dims):
 
 
 def _check(state, leaves, n, dims):
-    """_match, or what is wrong: the leaves walked one by one for the message."""
-    return _match(state, leaves, n, dims) or _check_leaves(leaves, n, dims)
+    """_match on a GPU, or what is wrong: the leaves walked one by one for the message."""
+    found = _match(state, leaves, n, dims)
+    return found if found and leaves[0].device.type == "cuda" else _check_leaves(leaves, n, dims)
 
 
 def _check_leaves(leaves, n, dims):

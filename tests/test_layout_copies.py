@@ -55,6 +55,19 @@ def test_clone_keeps_autograd_on_the_gpu(n):
     _grad_flows("cuda", n)
 
 
+@pytest.mark.parametrize("n,pitch", [(3, None), (64, None), (5, 9)])
+def test_clone_keeps_a_tangent(n, pitch):
+    """Inside a forward-mode level a leaf's tangent is copied with it."""
+    _, _, st, _ = _host_state(n)
+    dev = b2.layout.to_device(st, "cpu", pitch)
+    with torch.autograd.forward_ad.dual_level():
+        v = torch.autograd.forward_ad.make_dual(dev.bodies.v, torch.full_like(dev.bodies.v, 2.0))
+        out = b2.layout.clone(dev._replace(bodies=dev.bodies._replace(v=v)))
+        got = torch.autograd.forward_ad.unpack_dual(out.bodies.v)
+        assert got.tangent is not None and bool((got.tangent == 2.0).all())
+        assert torch.equal(got.primal, dev.bodies.v)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("case", ["one", "odd", "pitch", "leaves", "elsewhere", "batch_major", "double"])
 def test_clone_and_step_on_the_gpu(oracle, case):
