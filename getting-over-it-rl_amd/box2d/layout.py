@@ -52,6 +52,13 @@ def _spec(n, dims, pitch):
     return dtypes, shapes, strides, offsets[:-1], offsets[-1]
 
 
+def _traced():
+    """Whether the operations are recorded or rewritten (a dispatch mode, a functorch transform, torch.jit.trace,
+    torch.compile): one buffer's leaves alias it in ways those do not follow, so each leaf is then a tensor by itself."""
+    return (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() > 0
+            or torch._C._functorch.peek_interpreter_stack() is not None)
+
+
 def _carve(buf, n, dims, pitch):
     """The State whose leaves are the consecutive parts of the byte buffer buf. Each float leaf is a tensor of its own to
     autograd (.data): as views of one float tensor, a write that requires grad into one would make the next write into
@@ -67,10 +74,10 @@ def empty_device_state(n, dims, device="cuda", pitch=None, packed=True):
     """An uninitialised device State of n worlds with capacities dims = (B, R, J, C), pitch n by default. The leaves
     are by default the consecutive parts of one buffer, which a clone copies whole; with a pitch that is a multiple of
     64 that is the packed layout, which lets the step address every leaf from one base pointer. packed=False gives one
-    buffer per leaf."""
+    buffer per leaf, and so does code that is traced (_traced)."""
     pitch = n if pitch is None else pitch
     dims = tuple(dims)
-    if packed and pitch > 0:
+    if packed and pitch > 0 and not _traced():
         return _carve(torch.empty(_spec(n, dims, pitch)[4], dtype=torch.uint8, device=device), n, dims, pitch)
     vals = []
     for _, _, dt, inner in wd.LEAVES:
@@ -122,8 +129,10 @@ def clone_view(state):
 
 def _memory_is_all(leaves):
     """Whether a copy of the leaves' memory copies all they are. A leaf that requires grad is copied as a leaf, so that its
-    copy has it as its gradient's source, and so is every leaf inside a forward-mode level, where it may have a tangent."""
-    return forward_ad._current_level < 0 and not any(map(_REQUIRES_GRAD, leaves))
+    copy has it as its gradient's source, and so is every leaf inside a forward-mode level, where it may have a tangent,
+    of a tensor subclass, which may see the copy, and in traced code."""
+    return (not _traced() and forward_ad._current_level < 0 and not any(map(_REQUIRES_GRAD, leaves))
+            and list(map(type, leaves)) == [torch.Tensor] * len(leaves))
 
 
 def _copy_buffer(leaves, n, dims, pitch, ptrs):

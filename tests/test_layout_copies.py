@@ -68,6 +68,41 @@ def test_clone_keeps_a_tangent(n, pitch):
         assert torch.equal(got.primal, dev.bodies.v)
 
 
+@pytest.mark.parametrize("n", [3, 64])
+@pytest.mark.parametrize("how", ["make_fx", "functionalize", "jit", "compile"])
+def test_clone_is_traced(n, how):
+    """A traced clone copies its inputs at every call, not those that it was traced with."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    def ones(k):
+        return [t.fill_(k) for t in wd.leaves(b2.layout.to_device(_host_state(n)[2], "cpu"))]  # parts of one buffer
+
+    def copy(*leaves):
+        return tuple(wd.leaves(b2.layout.clone(wd.from_leaves(list(leaves)))))
+
+    traced = {"make_fx": lambda: make_fx(copy)(*ones(0)), "functionalize": lambda: torch.func.functionalize(copy),
+              "jit": lambda: torch.jit.trace(copy, tuple(ones(0)), check_trace=False),
+              "compile": lambda: torch.compile(copy, backend="eager")}[how]()
+    given = ones(1)
+    got = traced(*given)
+    assert all(torch.equal(a, b) and a.data_ptr() != b.data_ptr() for a, b in zip(got, given))
+
+
+def test_clone_of_a_subclass():
+    """A leaf of a tensor subclass sees its copy."""
+    class Seen(torch.Tensor):
+        calls = []
+
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            cls.calls.append(func.__name__)
+            return super().__torch_function__(func, types, args, kwargs or {})
+
+    dev = b2.layout.to_device(_host_state(3)[2], "cpu")
+    b2.layout.clone(dev._replace(bodies=dev.bodies._replace(v=dev.bodies.v.as_subclass(Seen))))
+    assert "copy_" in Seen.calls
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("case", ["one", "odd", "pitch", "leaves", "elsewhere", "batch_major", "double"])
 def test_clone_and_step_on_the_gpu(oracle, case):
