@@ -60,14 +60,14 @@ def _traced():
 
 
 def _carve(buf, n, dims, pitch):
-    """The State whose leaves are the consecutive parts of the byte buffer buf. Each float leaf is a tensor of its own to
-    autograd (.data): as views of one float tensor, a write that requires grad into one would make the next write into
-    any other an error."""
+    """The State whose leaves are the consecutive parts of the byte buffer buf. Each leaf is a tensor of its own to autograd
+    (.data, then its shape set in place): as views of one tensor they would share its version counter and its graph, so
+    that a write into one leaf spoiled what a backward pass saved of another."""
     dtypes, shapes, strides, offsets, _ = _spec(n, dims, pitch)
     typed = {torch.float32: buf.view(torch.float32), torch.int32: buf.view(torch.int32), torch.bool: buf.view(torch.bool)}
     size = {torch.float32: 4, torch.int32: 4, torch.bool: 1}
-    parts = [typed[dt].as_strided(sh, st, off // size[dt]) for dt, sh, st, off in zip(dtypes, shapes, strides, offsets)]
-    return wd.from_leaves([t.data if dt is torch.float32 else t for dt, t in zip(dtypes, parts)])
+    return wd.from_leaves([typed[dt].data.as_strided_(sh, st, off // size[dt])
+                           for dt, sh, st, off in zip(dtypes, shapes, strides, offsets)])
 
 
 def empty_device_state(n, dims, device="cuda", pitch=None, packed=True):

@@ -55,6 +55,30 @@ def test_clone_keeps_autograd_on_the_gpu(n):
     _grad_flows("cuda", n)
 
 
+@pytest.mark.parametrize("n", [3, 64])
+@pytest.mark.parametrize("copied", [False, True])
+def test_a_write_into_a_leaf_leaves_the_others(n, copied):
+    """A backward pass may use what it saved of a leaf (a mask, an index, a factor) after another leaf was written."""
+    dev = b2.layout.to_device(_host_state(n)[2], "cpu")
+    dev = b2.layout.clone(dev) if copied else dev
+    x = torch.ones(n, dev.contacts.touching.shape[1], requires_grad=True)
+    mask, at, by = dev.contacts.touching, dev.contacts.count, dev.contacts.friction
+    versions = [t._version for t in wd.leaves(dev)]
+    loss = (torch.where(mask, x, 2 * x) + x[torch.arange(n)[:, None], at.long()] + x * by).sum()
+    for leaf in (dev.new_fixture, dev.next_key, dev.bodies.v):
+        leaf.zero_()
+    loss.backward()
+    assert x.grad is not None
+    written = {k for k, t in enumerate(wd.leaves(dev)) if t._version != versions[k]}
+    assert written == {k for k, t in enumerate(wd.leaves(dev)) if any(t is w for w in (dev.new_fixture, dev.next_key,
+                                                                                       dev.bodies.v))}
+
+
+def test_leaves_in_inference_mode():
+    with torch.inference_mode():
+        _copies(b2.layout.to_device(_host_state(3)[2], "cpu"), _host_state(3)[2])
+
+
 @pytest.mark.parametrize("n,pitch", [(3, None), (64, None), (5, 9)])
 def test_clone_keeps_a_tangent(n, pitch):
     """Inside a forward-mode level a leaf's tangent is copied with it."""
