@@ -137,10 +137,13 @@ def _memory_is_all(leaves):
 
 def _copy_buffer(leaves, n, dims, pitch, ptrs):
     """A copy of the one buffer whose consecutive parts the (checked) leaves are, by a single device copy, or None where
-    the leaves are not laid out so."""
+    the leaves are not laid out so, or are the first few worlds of a much larger buffer: the copy holds all of it, so more
+    padding than worlds is copied only up to 1 MiB (16 of 65,536 rig worlds would hold 373 MB)."""
     if pitch <= 0:
         return None
     _, _, _, offsets, nbytes = _spec(n, dims, pitch)
+    if pitch > 2 * n and nbytes > 1 << 20:
+        return None
     base = ptrs[0]
     if ptrs != [base + o for o in offsets]:
         return None

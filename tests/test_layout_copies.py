@@ -55,6 +55,20 @@ def test_clone_keeps_autograd_on_the_gpu(n):
     _grad_flows("cuda", n)
 
 
+@pytest.mark.parametrize("n,k,whole", [(4096, 16, False), (4096, 2047, False), (4096, 2048, True), (64, 1, True)])
+def test_clone_of_the_first_worlds(n, k, whole):
+    """A State narrowed to its first worlds: the copy holds what those need, not the State that they are part of (whose
+    padding is copied along where it is no more than the worlds, or small)."""
+    one = _host_state(1)[2]
+    dev = b2.layout.empty_device_state(n, wd.dims(one), "cpu")
+    for dst, src in zip(wd.leaves(dev), wd.leaves(one)):
+        dst.copy_(torch.from_numpy(np.ascontiguousarray(src)).expand(dst.shape))
+    out = _copies(wd.from_leaves([t[:k] for t in wd.leaves(dev)]), wd.batch(wd.from_leaves([x[0] for x in wd.leaves(one)]), k))
+    held = sum({t.untyped_storage().data_ptr(): t.untyped_storage().nbytes() for t in wd.leaves(out)}.values())
+    need = 4 * b2.layout.packed_words(wd.dims(one))[-1]
+    assert held == need * (n if whole else k)
+
+
 @pytest.mark.parametrize("n", [3, 64])
 @pytest.mark.parametrize("copied", [False, True])
 def test_a_write_into_a_leaf_leaves_the_others(n, copied):
