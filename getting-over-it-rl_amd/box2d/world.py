@@ -8,6 +8,7 @@ Indices follow creation order, which Box2D uses for its orderings (world.py:7-11
 body list is newest first, so islands are seeded from the highest index); fixture i gets broad-phase proxy id order i;
 joint i is the i-th created (each body's joint list is newest first).
 """
+import itertools
 from dataclasses import dataclass
 from typing import NamedTuple
 
@@ -213,7 +214,8 @@ def leaves(state):
 
 
 def from_leaves(vals):
-    """A State from 71 leaves in ABI order."""
+    """A State from 71 leaves in ABI order: the first 71 of any iterable."""
+    vals = list(itertools.islice(vals, len(LEAVES)))
     i = [0]
     for part in (Bodies, Fixtures, Joints, Contacts):
         i.append(i[-1] + len(part._fields))

@@ -95,6 +95,15 @@ def test_state_fields_follow_reference_pytree():
     assert wd.ContactTOI._fields[-1] == "events"
 
 
+def test_from_leaves_takes_any_iterable():
+    """The first 71 values of a list, an iterator or a longer sequence, in ABI order."""
+    vals = list(range(len(wd.LEAVES)))
+    want = wd.from_leaves(vals)
+    assert wd.leaves(want) == vals
+    for given in (iter(vals), (x for x in vals), tuple(vals), vals + [-1, -2], dict.fromkeys(vals)):
+        assert wd.from_leaves(given) == want
+
+
 def test_model_fields_extend_the_reference_model():
     """The reference's Model fields in its order (world.py:30-65), then this package's additions, so a Model built
     positionally or by keyword for the reference is accepted."""
