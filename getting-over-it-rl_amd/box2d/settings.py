@@ -85,7 +85,10 @@ class Settings:
     def to_c(self):
         """The C ABI struct (include/goi_b2.h GoiSettings)."""
         from ._abi import GoiSettings
-        f = lambda n: getattr(self, n)  # noqa: E731  (a c_float field rounds as F32 does)
+
+        def f(name):
+            v = getattr(self, name)  # a c_float field rounds as F32 does, but takes fewer kinds of value (no text)
+            return v if type(v) is F32 or type(v) is float else float(F32(v))
         return GoiSettings(
             velocity_iterations=int(self.velocity_iterations), position_iterations=int(self.position_iterations),
             linear_slop=f("linear_slop"), angular_slop=f("angular_slop"), polygon_radius=f("polygon_radius"),

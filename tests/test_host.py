@@ -69,6 +69,14 @@ def test_settings_to_c_round_trip():
     assert b2.Settings.stock().to_c().max_events == -1
 
 
+@pytest.mark.parametrize("value", [0.1, F32(0.1), np.float64(0.1), "0.1", "1e-1", np.array(0.1), 1, True, 0.1 + 1e-9])
+def test_settings_to_c_rounds_like_float32(value):
+    """A float setting is what float32 makes of the value, text from a configuration file included."""
+    assert b2.Settings(baumgarte=value).to_c().baumgarte == float(F32(value))
+    with pytest.raises((TypeError, ValueError)):
+        b2.Settings(baumgarte="half").to_c()
+
+
 # ---------------------------------------------------------------------------------------------------------------
 # the leaf table and the header
 
