@@ -104,7 +104,9 @@ def _launch(model, state, view, settings, dt, n, debug, stream):
     cs = settings.to_c()
     st = torch.cuda.current_stream(dev).cuda_stream if stream is None else stream
     dbg = None if debug is None else ctypes.byref(debug)
-    _abi.check(dm.L.goi_step_n(dm.handle, ctypes.byref(view), ctypes.byref(cs), np.float32(dt), n, st, dbg), dm.L)
+    # c_void_p takes an integer or None only; as the bare argument, bytes would pass as their own address
+    _abi.check(dm.L.goi_step_n(dm.handle, ctypes.byref(view), ctypes.byref(cs), np.float32(dt), n, ctypes.c_void_p(st),
+                               dbg), dm.L)
 
 
 def _need_hip(settings):

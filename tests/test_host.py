@@ -345,6 +345,29 @@ def test_bad_arguments_fail_before_the_device():
     assert L.goi_last_launch(ctypes.byref(info)) == A.GOI_OK and info.kernel == 0  # nothing launched here
 
 
+def test_stream_is_a_handle(monkeypatch):
+    """step_'s stream is an integer handle (hipStream_t) or 0; anything else is refused before the library sees it."""
+    import importlib
+    A, step = abi(), importlib.import_module(b2.__name__ + ".step")
+    seen = []
+    fn = ctypes.CFUNCTYPE(ctypes.c_int32, *[ctypes.c_void_p] * 3, ctypes.c_float, ctypes.c_int32, ctypes.c_void_p,
+                          ctypes.c_void_p)(lambda *a: seen.append(a[5]) or 0)
+    fn.argtypes = [ctypes.c_void_p, ctypes.POINTER(A.GoiStateView), ctypes.POINTER(A.GoiSettings), ctypes.c_float,
+                   ctypes.c_int32, ctypes.c_void_p, ctypes.POINTER(A.GoiDebug)]
+    stub = type("Stub", (), {"L": type("L", (), {"goi_step_n": staticmethod(fn)}), "handle": None})
+    monkeypatch.setattr(step, "device_model", lambda *a, **k: stub)
+    s, m, st, cfg = b2.scenes.make_config(1, 1)
+    dev = b2.layout.to_device(st, "cpu")
+    args = m, dev, A.GoiStateView(), s, cfg.dt, 1, None
+    step._launch(*args, 0)
+    step._launch(*args, 0x1234)
+    assert seen == [None, 0x1234]
+    for bad in (b"stream", "stream", object(), type("S", (), {"_as_parameter_": ctypes.c_void_p(8)})()):
+        with pytest.raises(TypeError):
+            step._launch(*args, bad)
+    assert len(seen) == 2
+
+
 def test_host_state_is_rejected():
     """The step runs on device States only: numpy or CPU tensors raise before anything reaches the library."""
     s, m, st, cfg = b2.scenes.make_config(1, 2)
