@@ -142,12 +142,15 @@ GOI_D void jn_prepare(const DModel& m, const World& W, const Bodies& bd, const R
 }
 
 // the velocity part of InitVelocityConstraints (joints.py:202-248)
-GOI_D void jn_warm_start(const Bodies& bd, const Rows& R, int i, bool v24, bool rev_only) {
+template <class BD>
+GOI_D void jn_warm_start(const BD& bd, const Rows& R, int i, bool v24, bool rev_only) {
     const int type = rev_only ? (int)GOI_REVOLUTE : R.geti(i, JF_TYPE), ia = R.geti(i, JF_IA), ib = R.geti(i, JF_IB);
     const float mA = R.getf(i, JF_MA), mB = R.getf(i, JF_MB), iA = R.getf(i, JF_IIA), iB = R.getf(i, JF_IIB);
     const float ix = R.getf(i, JF_IMP0), iy = R.getf(i, JF_IMP1), iz = R.getf(i, JF_IMP2), mi = R.getf(i, JF_MIMP);
-    V2 vA = bd.v(ia), vB = bd.v(ib);
-    float wA = bd.w(ia), wB = bd.w(ib);
+    const V2 vA0 = bd.v(ia), vB0 = bd.v(ib);
+    const float wA0 = bd.w(ia), wB0 = bd.w(ib);
+    V2 vA = vA0, vB = vB0;
+    float wA = wA0, wB = wB0;
     if (type == GOI_PRISMATIC) {
         const float mz = mi + iz;
         const V2 P = ix * R.get2(i, JF_PX) + mz * R.get2(i, JF_AX);
@@ -172,12 +175,13 @@ GOI_D void jn_warm_start(const Bodies& bd, const Rows& R, int i, bool v24, bool 
             wB = wB + iB * (cross(rB, P) + iz);
         }
     }
-    bd.set_v(ia, vA, wA);
-    bd.set_v(ib, vB, wB);
+    bd.set_v(ia, vA, wA, vA0, wA0);
+    bd.set_v(ib, vB, wB, vB0, wB0);
 }
 
 // SolveVelocityConstraints for joint row i (joints.py:257-437, revolute24.patch:166-240)
-GOI_D void jn_solve_velocity(const Bodies& bd, const Rows& R, int i, bool v24, bool rev_only) {
+template <class BD>
+GOI_D void jn_solve_velocity(const BD& bd, const Rows& R, int i, bool v24, bool rev_only) {
     const int type = rev_only ? (int)GOI_REVOLUTE : R.geti(i, JF_TYPE), ia = R.geti(i, JF_IA), ib = R.geti(i, JF_IB);
     const float mA = R.getf(i, JF_MA), mB = R.getf(i, JF_MB), iA = R.getf(i, JF_IIA), iB = R.getf(i, JF_IIB);
     const bool emotor = R.geti(i, JF_EMOTOR) != 0, elimit = R.geti(i, JF_ELIMIT) != 0;
@@ -190,8 +194,10 @@ GOI_D void jn_solve_velocity(const Bodies& bd, const Rows& R, int i, bool v24, b
     const V2 jrA = R.get2(i, JF_RA), jrB = R.get2(i, JF_RB);
     const float jangle = R.getf(i, JF_ANGLE), jinv_dt = R.getf(i, JF_INVDT);
     const float jlower = R.getf(i, JF_LOWER), jupper = R.getf(i, JF_UPPER);
-    V2 vA = bd.v(ia), vB = bd.v(ib);
-    float wA = bd.w(ia), wB = bd.w(ib);
+    const V2 vA0 = bd.v(ia), vB0 = bd.v(ib);
+    const float wA0 = bd.w(ia), wB0 = bd.w(ib);
+    V2 vA = vA0, vB = vB0;
+    float wA = wA0, wB = wB0;
     if (type == GOI_REVOLUTE) {
         const V2 rA = jrA, rB = jrB;
         const bool fixed = (iA + iB) == 0.0f;
@@ -323,8 +329,8 @@ GOI_D void jn_solve_velocity(const Bodies& bd, const Rows& R, int i, bool v24, b
     }
     R.setf(i, JF_IMP0, i0); R.setf(i, JF_IMP1, i1); R.setf(i, JF_IMP2, i2);
     R.setf(i, JF_IMP3, i3); R.setf(i, JF_IMP4, i4); R.setf(i, JF_MIMP, mi);
-    bd.set_v(ia, vA, wA);
-    bd.set_v(ib, vB, wB);
+    bd.set_v(ia, vA, wA, vA0, wA0);
+    bd.set_v(ib, vB, wB, vB0, wB0);
 }
 
 // A revolute joint's row under the v2.4.1 solver (revolute24.patch:78-330, joints.py:61-520), set up by the lane that
@@ -397,7 +403,8 @@ GOI_D void warm_rev_row(const LaneBodies& bd, const RevRow& r) {
     bd.set_v(r.ia, vA, wA, vA0, wA0);
     bd.set_v(r.ib, vB, wB, vB0, wB0);
 }
-GOI_D void solve_rev_row(const LaneBodies& bd, RevRow& r) {
+template <class BD>
+GOI_D void solve_rev_row(const BD& bd, RevRow& r) {
     const V2 vA0 = bd.v(r.ia), vB0 = bd.v(r.ib);
     const float wA0 = bd.w(r.ia), wB0 = bd.w(r.ib);
     V2 vA = vA0, vB = vB0;
@@ -437,6 +444,50 @@ GOI_D void solve_rev_row(const LaneBodies& bd, RevRow& r) {
     bd.set_v(r.ia, vA, wA, vA0, wA0);
     bd.set_v(r.ib, vB, wB, vB0, wB0);
 }
+// the velocity-solver fields of row i of the row tile, loaded in one batch (jn_prepare's; 1 / det is not in it)
+GOI_D RevRow load_rev_row(const Rows& R, int i) {
+    RevRow r;
+    r.ia = R.geti(i, JF_IA); r.ib = R.geti(i, JF_IB);
+    r.emotor = R.geti(i, JF_EMOTOR) != 0; r.elimit = R.geti(i, JF_ELIMIT) != 0;
+    r.mA = R.getf(i, JF_MA); r.mB = R.getf(i, JF_MB); r.iA = R.getf(i, JF_IIA); r.iB = R.getf(i, JF_IIB);
+    r.k11 = R.getf(i, JF_EXX); r.k21 = R.getf(i, JF_EXX + 1); r.k12 = R.getf(i, JF_EYX); r.k22 = R.getf(i, JF_EYX + 1);
+    r.i0 = R.getf(i, JF_IMP0); r.i1 = R.getf(i, JF_IMP1); r.i3 = R.getf(i, JF_IMP3); r.i4 = R.getf(i, JF_IMP4);
+    r.mi = R.getf(i, JF_MIMP);
+    r.maximp = R.getf(i, JF_MAXIMP); r.mspeed = R.getf(i, JF_MSPEED); r.mmass = R.getf(i, JF_MMASS);
+    r.rA = R.get2(i, JF_RA); r.rB = R.get2(i, JF_RB);
+    r.angle = R.getf(i, JF_ANGLE); r.inv_dt = R.getf(i, JF_INVDT);
+    r.lower = R.getf(i, JF_LOWER); r.upper = R.getf(i, JF_UPPER);
+    return r;
+}
+// row i's velocity solve from the tile
+template <class BD>
+GOI_D void solve_rev_tile_row(const BD& bd, const Rows& R, int i, RevRow& r) {
+    float det = r.k11 * r.k22 - r.k12 * r.k21;
+    if (det != 0.0f) det = fdiv(1.0f, det);
+    r.inv_det = det;
+    solve_rev_row(bd, r);
+    R.setf(i, JF_IMP0, r.i0); R.setf(i, JF_IMP1, r.i1);
+    R.setf(i, JF_IMP3, r.i3); R.setf(i, JF_IMP4, r.i4); R.setf(i, JF_MIMP, r.mi);
+}
+// joint rows i0 .. n-1 of the row tile once each, in order. A revolute-only model's rows under the v2.4.1 solver load one
+// ahead, two rows an iteration (as cs_solve_velocity_sweep).
+template <class BD>
+GOI_D void jn_solve_velocity_sweep(const BD& bd, const Rows& R, int i0, int n, bool v24, bool rev_only) {
+    if (!(rev_only && v24)) {
+        for (int i = i0; i < n; ++i) jn_solve_velocity(bd, R, i, v24, rev_only);
+        return;
+    }
+    if (n <= i0) return;
+    RevRow a = load_rev_row(R, i0), b;
+    for (int i = i0; i < n; i += 2) {
+        if (i + 1 < n) b = load_rev_row(R, i + 1);
+        solve_rev_tile_row(bd, R, i, a);
+        if (i + 1 >= n) break;
+        if (i + 2 < n) a = load_rev_row(R, i + 2);
+        solve_rev_tile_row(bd, R, i + 1, b);
+    }
+}
+
 GOI_D void store_rev_row(const World& W, const RevRow& r) {
     const int j = r.jid;
     W.f(GOI_J_IMPULSE, 3 * j) = r.i0;
@@ -514,7 +565,8 @@ GOI_D bool solve_rev_position(const LaneBodies& bd, const RevRow& r, const GoiSe
 }
 
 // SolvePositionConstraints for joint row i (joints.py:462-606); returns the joint's ok flag
-GOI_D bool jn_solve_position(const Bodies& bd, const Rows& R, int i, const GoiSettings& s, bool rev_only) {
+template <class BD>
+GOI_D bool jn_solve_position(const BD& bd, const Rows& R, int i, const GoiSettings& s, bool rev_only) {
     const int type = rev_only ? (int)GOI_REVOLUTE : R.geti(i, JF_TYPE), ia = R.geti(i, JF_IA), ib = R.geti(i, JF_IB);
     const float mA = R.getf(i, JF_MA), mB = R.getf(i, JF_MB), iA = R.getf(i, JF_IIA), iB = R.getf(i, JF_IIB);
     const bool elimit = R.geti(i, JF_ELIMIT) != 0;
@@ -524,8 +576,10 @@ GOI_D bool jn_solve_position(const Bodies& bd, const Rows& R, int i, const GoiSe
     const int jst = R.geti(i, JF_STATE);
     const V2 jla = R.get2(i, JF_LA), jlb = R.get2(i, JF_LB);
     const float mac = s.max_angular_correction;
-    V2 cA = bd.c(ia), cB = bd.c(ib);
-    float aA = bd.a(ia), aB = bd.a(ib);
+    const V2 cA0 = bd.c(ia), cB0 = bd.c(ib);
+    const float aA0 = bd.a(ia), aB0 = bd.a(ib);
+    V2 cA = cA0, cB = cB0;
+    float aA = aA0, aB = aB0;
     bool ok;
     if (type == GOI_REVOLUTE) {
         const bool fixed = (iA + iB) == 0.0f;
@@ -636,8 +690,8 @@ GOI_D bool jn_solve_position(const Bodies& bd, const Rows& R, int i, const GoiSe
         }
         ok = pos_err <= s.linear_slop && ang_err <= s.angular_slop;
     }
-    bd.set_c(ia, cA, aA);
-    bd.set_c(ib, cB, aB);
+    bd.set_c(ia, cA, aA, cA0, aA0);
+    bd.set_c(ib, cB, aB, cB0, aB0);
     return ok;
 }
 

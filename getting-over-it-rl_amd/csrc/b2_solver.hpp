@@ -85,6 +85,13 @@ struct Islands {
     GOI_D int& body_island(int b) const { return W.bisl(b); }
     GOI_D int& contact_island(int c) const { return W.cisl(c); }
     GOI_D int& joint_island(int j) const { return W.jisl(j); }
+    // island k's contact rows [c0, c1) and joint rows [j0, j1) of the solve order, where find_islands noted its starts
+    // (DModel::island_lanes)
+    GOI_D void rows_of(int k, int& c0, int& c1, int& j0, int& j1) const {
+        const int s0 = W.ibuf(k), s1 = k + 1 < n ? W.ibuf(k + 1) : (nc | (nj << 16));
+        c0 = s0 & 0xffff; j0 = s0 >> 16;
+        c1 = s1 & 0xffff; j1 = s1 >> 16;
+    }
 };
 
 // sets bits of a workspace word that several lanes of the group may set
@@ -132,6 +139,8 @@ GOI_D void find_islands(const DModel& m, const World& W, Islands& I) {
         if ((bflag >> seed) & 1ull) continue;
         if (!W.awake(seed) || !W.active(seed) || W.is_static(seed)) continue;
         const int isl = nisl++;
+        // the island's first rows (nc < 2^16, nj <= 64), in the solver's body words while ibuf holds masks
+        if (m.island_lanes) W.wi(W.k.o_body, isl) = nc | (nj << 16);
         int sp = 0;
         W.stack(sp++) = seed;
         bflag |= 1ull << seed;
@@ -188,6 +197,11 @@ GOI_D void find_islands(const DModel& m, const World& W, Islands& I) {
     I.nc = nc;
     I.nj = nj;
     I.n = nisl;
+    if (m.island_lanes) {
+        group_sync();
+        for (int k = W.sub; k < nisl; k += W.G) W.ibuf(k) = W.wi(W.k.o_body, k);
+        group_sync();
+    }
 }
 
 // ---------------------------------------------------------------- contact solver (contact_solver.py)
@@ -606,7 +620,8 @@ GOI_D void store_vimpulses(const Rows& R, int i, const VRow& r) {
 
 // rows i0..n-1 once each, in order, each loaded in one batch while the row before it is solved; two rows a loop
 // iteration, so the two row buffers alternate without copies between them
-GOI_D void cs_solve_velocity_sweep(const Bodies& bd, const Rows& R, int i0, int n) {
+template <class BD>
+GOI_D void cs_solve_velocity_sweep(const BD& bd, const Rows& R, int i0, int n) {
     if (n <= i0) return;
     VRow a = load_vrow(R, i0), b;
     for (int i = i0; i < n; i += 2) {

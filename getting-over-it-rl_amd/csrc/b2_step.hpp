@@ -17,7 +17,8 @@ namespace goi {
 // at once, on their lanes: each contact row has a level, one more than the highest level of the rows before it that
 // share one of its moving bodies, and an iteration runs the levels in order. Every row then sees the bodies as it does
 // in the sequential order (LaneBodies has the static bodies' side of that), so the results are the same floats.
-// Joints keep their sequential order, one after another (the rig's form one chain). Measured on the 4-body rig: a
+// Joint rows run in levels of their own, before the contacts' (10 rigs a world, 1,000 worlds at 300 / 30 iterations: 3.4
+// ms a step with the joints one after another, 1.03 in levels). Measured on the 4-body rig: a
 // velocity iteration of 3 joints and 1 contact on a wave of its own 1.66 -> 1.15 us; the 8 iterations of 8 worlds a
 // wave 34 -> 16.5 us; a step at 300 / 30 iterations of 1,024 worlds 2.82 -> 1.15 ms.
 // A second row a lane costs registers (spills, 3% of a step at 2 worlds per wave), so only groups of up to 16 lanes have
@@ -38,8 +39,11 @@ struct LaneContacts {
 };
 struct LaneJoints {
     RevRow r[kLaneJoints];
-    int at[kLaneJoints];  // the row's place in the solve order, -1: no row
-    bool pair, odd;       // two lanes hold each row; this is the second
+    int level[kLaneJoints];  // -1: no row
+    int levels;              // the world's
+    bool pair, odd;          // two lanes hold each row; this is the second
+    // the place in the solve order of the lane's row k
+    GOI_D int at(const World& W, int k) const { return (W.sub + k * W.G) >> (pair ? 1 : 0); }
 };
 
 // The lane's contact rows' slots and levels. The last level of each body (0: none yet) is in the search's stack, which
@@ -80,21 +84,127 @@ GOI_D void by_level(const LaneContacts& lc, F&& f) {
         group_sync();  // the bodies one lane wrote are read by others in the next level
     }
 }
-// f(k) for the lane's joint rows, in the solve order
-template <class F>
-GOI_D void in_order(const LaneJoints& lj, int nj, F&& f) {
-    for (int i = 0; i < nj; ++i) {
+// The lane's joint rows' levels: in a world of one island the solve order itself (the joints there mostly form a chain,
+// which has no two rows to run at once), else as lane_levels, the rows' bodies coming from the lanes that hold them.
+GOI_D void joint_levels(const DModel& m, const World& W, const Islands& I, LaneJoints& lj) {
+#pragma unroll
+    for (int k = 0; k < kLaneJoints; ++k) lj.level[k] = lj.at(W, k) < I.nj ? lj.at(W, k) : -1;
+    lj.levels = I.nj;
+    if (!m.island_lanes || I.n <= 1) return;
+    for (int b = W.sub; b < W.B; b += W.G) W.stack(b) = 0;
+    group_sync();
+    lj.levels = 0;
+    for (int i = 0; i < I.nj; ++i) {
+        const int at = lj.pair ? 2 * i : i;
+        int a = 0, b = 0;
+#pragma unroll
+        for (int k = 0; k < kLaneJoints; ++k) {
+            if (at < k * W.G || at >= (k + 1) * W.G) continue;
+            a = group_lane(W.grp(), lj.r[k].ia, at - k * W.G);
+            b = group_lane(W.grp(), lj.r[k].ib, at - k * W.G);
+        }
+        const bool fa = W.is_static(a), fb = W.is_static(b);
+        const int level = max(fa ? 0 : W.stack(a), fb ? 0 : W.stack(b));
+        if (!fa) W.stack(a) = level + 1;
+        if (!fb) W.stack(b) = level + 1;
+        lj.levels = max(lj.levels, level + 1);
 #pragma unroll
         for (int k = 0; k < kLaneJoints; ++k)
-            if (lj.at[k] == i) f(k);
+            if (lj.at(W, k) == i) lj.level[k] = level;
+    }
+    group_sync();
+}
+// f(k) for the lane's joint rows, level by level
+template <class F>
+GOI_D void by_level(const LaneJoints& lj, F&& f) {
+    for (int l = 0; l < lj.levels; ++l) {
+#pragma unroll
+        for (int k = 0; k < kLaneJoints; ++k)
+            if (lj.level[k] == l) f(k);
         group_sync();
     }
 }
 
 // Whether the group's registers hold the world's rows: every contact row, and every joint row as a RevRow.
 GOI_D bool rows_fit(const DModel& m, const World& W, const Islands& I, const GoiSettings& s) {
-    return I.nc <= kLaneRows * W.G && I.nj <= kLaneJoints * W.G && m.rev_only && s.revolute_v24 &&
+    return I.nc <= kLaneRows * W.G && (I.nj == 0 || (I.nj <= kLaneJoints * W.G && m.rev_only && s.revolute_v24)) &&
            s.linear_slop >= 0.0f;
+}
+
+// ---- Solve on the row tiles
+//
+// A world whose rows the registers do not hold (more rows, other joints, the v2.3.1 solver) takes them from the row
+// tiles. Where it has several islands (kIslands), its group's lanes solve them side by side, each its own: islands share
+// no body but static ones (island.py:3-7; LaneBodies has those bodies' side of it). One after another, the islands'
+// chains add up: ms a step at 300 / 30 iterations, in turn -> side by side: 8 prismatic pairs a world, 512 worlds, 5.3 ->
+// 1.8; 6 rigs a world, 8,192 worlds at 4 a wave (18 joints on 16 lanes), 15.7 -> 6.2; 6 rigs under the v2.3.1 solver,
+// 1,500 worlds, 8.2 -> 2.0.
+
+// How a world's rows are solved. If a row would change a static body, the velocity phase runs again from the integration,
+// row after row (kRows), as does the position phase from the integrated poses (kPositions).
+enum Solve { kLanes, kIslands, kRows, kPositions, kSolved };
+
+// b2Island::Solve's warm start and velocity iterations (step.py:96-117) on the row tiles: the lane's islands, or (kRows)
+// all rows in order, by every lane. False when a static body would have changed (nothing but bd and the tiles is written).
+GOI_D bool tile_velocities(const DModel& m, const World& W, const Bodies& bd, const Rows& CR, const Rows& JRw,
+                           const Islands& I, const GoiSettings& s, bool islands) {
+    const bool v24 = s.revolute_v24 != 0;
+    unsigned changed = 0u;
+    const LaneBodies lb{bd, islands ? W.smask : 0ull, &changed};
+    for (int k = islands ? W.sub : 0; k < (islands ? I.n : 1); k += W.G) {
+        int c0 = 0, c1 = I.nc, j0 = 0, j1 = I.nj;
+        if (islands) I.rows_of(k, c0, c1, j0, j1);
+        if (s.warm_starting)
+            for (int i = c0; i < c1; ++i) warm_vrow(lb, load_vrow(CR, i));
+        for (int i = j0; i < j1; ++i) jn_warm_start(lb, JRw, i, v24, m.rev_only);
+        for (int it = 0; it < s.velocity_iterations; ++it) {
+            jn_solve_velocity_sweep(lb, JRw, j0, j1, v24, m.rev_only);
+            cs_solve_velocity_sweep(lb, CR, c0, c1);
+        }
+    }
+    group_sync();
+    return !group_any(W.grp(), changed != 0u);
+}
+
+// The position iterations (step.py:197-251) on the row tiles, by the same lanes, each island stopping at its first pass
+// within tolerance; returns the islands that did. `ok` is cleared when a static body would have changed or a separation
+// was NaN.
+GOI_D unsigned long long tile_positions(const DModel& m, const World& W, const Bodies& bd, const Rows& CR,
+                                        const Rows& JRw, const Islands& I, const GoiSettings& s, bool islands, bool& ok) {
+    const float okay_sep = -3.0f * s.linear_slop;
+    unsigned changed = 0u;
+    const LaneBodies lb{bd, islands ? W.smask : 0ull, &changed};
+    unsigned long long done = 0ull;
+    RotMemo qa, qb;
+    for (int k = islands ? W.sub : 0; k < (islands ? I.n : 1); k += W.G) {
+        int c0 = 0, c1 = I.nc, j0 = 0, j1 = I.nj;
+        const int n0 = islands ? k : 0, n1 = islands ? k + 1 : I.n;
+        if (islands) I.rows_of(k, c0, c1, j0, j1);
+        for (int it = 0, left = n1 - n0; it < s.position_iterations && left > 0; ++it) {
+            unsigned long long jbad = 0ull;
+            for (int i = n0; i < n1; ++i) W.fwork(i) = 0.0f;  // min separation per island
+            for (int i = c0; i < c1; ++i) {
+                const int isl = I.contact_island(I.corder(i));
+                if ((done >> isl) & 1ull) continue;
+                const PRow r = load_prow(CR, i);
+                W.fwork(isl) = bmin(W.fwork(isl), solve_prow(lb, r, s.baumgarte, r.mA, r.mB, r.iA, r.iB, s.linear_slop,
+                                                             s.max_linear_correction, qa, qb));
+            }
+            for (int i = j0; i < j1; ++i) {
+                const int isl = I.joint_island(JRw.geti(i, JF_JID));
+                if ((done >> isl) & 1ull) continue;
+                if (!jn_solve_position(lb, JRw, i, s, m.rev_only)) jbad |= 1ull << isl;
+            }
+            for (int i = n0; i < n1; ++i)
+                if (!((done >> i) & 1ull) && W.fwork(i) >= okay_sep && !((jbad >> i) & 1ull)) {
+                    done |= 1ull << i;
+                    --left;
+                }
+        }
+    }
+    group_sync();
+    ok = !group_any(W.grp(), changed != 0u);
+    return group_or(W.grp(), done);
 }
 
 // The world's rows set up in its lanes' registers, the warm start and the velocity iterations, and StoreImpulses.
@@ -118,17 +228,17 @@ GOI_D bool solve_velocities(const DModel& m, const World& W, const Bodies& bd, c
     lj.odd = lj.pair && (W.sub & 1);
 #pragma unroll
     for (int k = 0; k < kLaneJoints; ++k) {
-        const int i = lj.pair ? (W.sub + k * W.G) >> 1 : W.sub + k * W.G;
-        lj.at[k] = i < I.nj ? i : -1;
-        if (lj.at[k] < 0) continue;
+        const int i = lj.at(W, k);
+        if (i >= I.nj) continue;
         lj.r[k] = rev_row_of(m, W, bd, I.jorder(i), s, dt, dt_ratio, warm);
         lj.r[k].isl = I.joint_island(lj.r[k].jid);
     }
+    joint_levels(m, W, I, lj);
     group_sync();
     if (warm) by_level(lc, [&](int k) { warm_vrow(lb, lc.v[k]); });
-    in_order(lj, I.nj, [&](int k) { warm_rev_row(lb, lj.r[k]); });
+    by_level(lj, [&](int k) { warm_rev_row(lb, lj.r[k]); });
     for (int it = 0; it < s.velocity_iterations; ++it) {
-        in_order(lj, I.nj, [&](int k) { solve_rev_row(lb, lj.r[k]); });
+        by_level(lj, [&](int k) { solve_rev_row(lb, lj.r[k]); });
         by_level(lc, [&](int k) { solve_vrow(lb, lc.v[k]); });
     }
     if (group_any(W.grp(), changed != 0u)) return false;
@@ -147,7 +257,7 @@ GOI_D bool solve_velocities(const DModel& m, const World& W, const Bodies& bd, c
     }
 #pragma unroll
     for (int k = 0; k < kLaneJoints; ++k)
-        if (lj.at[k] >= 0) store_rev_row(W, lj.r[k]);
+        if (lj.level[k] >= 0) store_rev_row(W, lj.r[k]);
     return true;
 }
 
@@ -178,7 +288,7 @@ GOI_D bool solve_positions(const DModel& m, const World& W, const Bodies& bd, co
                                          s.max_linear_correction, qa[k], qb[k]);
             if (!(sep >= okay_sep)) bad |= 1ull << isl[k];
         });
-        in_order(lj, I.nj, [&](int k) {
+        by_level(lj, [&](int k) {
             if ((done >> lj.r[k].isl) & 1ull) return;
             if (!solve_rev_position(lb, lj.r[k], s, lj.pair, lj.odd)) bad |= 1ull << lj.r[k].isl;
         });
@@ -190,105 +300,47 @@ GOI_D bool solve_positions(const DModel& m, const World& W, const Bodies& bd, co
         if (lc.level[k] >= 0) store_prow(CR, W.sub + k * W.G, lc.slot[k], p[k]);
 #pragma unroll
     for (int k = 0; k < kLaneJoints; ++k)
-        if (lj.at[k] >= 0) store_rev_prow(JRw, lj.at[k], lj.r[k]);
+        if (lj.level[k] >= 0) store_rev_prow(JRw, lj.at(W, k), lj.r[k]);
     group_sync();
     return false;
 }
 
-GOI_D void solve_world(const DModel& m, const World& W, const Bodies& bd, const Rows& CR, const Rows& JRw,
-                            const GoiSettings& s, float dt, const GoiDebug& dbg) {
-    const float dt_ratio = W.f(GOI_S_INV_DT0, 0) * dt;
-    Islands I{W, 0, 0, 0};
-    find_islands(m, W, I);
-    const float h = dt;
+// The bodies' solver words as Solve begins: velocities of dynamic island bodies integrated (the sweep starts at the
+// current pose), poses and their rotations. Bodies are independent here and in the other per-body loops below: one body
+// per lane of the group.
+GOI_D void integrate_velocities(const World& W, const Bodies& bd, const Islands& I, float h) {
     const float gx = W.f(GOI_S_GRAVITY, 0), gy = W.f(GOI_S_GRAVITY, 1);
-    const bool warm = s.warm_starting != 0;
-    const bool v24 = s.revolute_v24 != 0;
-    // The rows in the lanes' registers where they fit. If a row would change a static body, the velocity phase runs
-    // again from the integration below on rows in the row tiles, one after another, as does the position phase from
-    // the integrated poses.
-    bool lanes = rows_fit(m, W, I, s);
-    LaneContacts lc;
-    LaneJoints lj;
-    for (;;) {
-        // integrate velocities of dynamic island bodies; the sweep starts at the current pose (bodies are independent
-        // here and in the other per-body loops below: one body per lane of the group)
-        for (int b = W.sub; b < W.B; b += W.G) {
-            V2 v = W.v2(GOI_B_V, b);
-            float w = W.f(GOI_B_W, b);
-            const V2 c = W.v2(GOI_B_C, b);
-            const float a = W.f(GOI_B_A, b);
-            if (I.body_island(b) >= 0) {
-                if (W.is_dynamic(b)) {
-                    const float gs = W.f(GOI_B_GRAVITY_SCALE, b), im = W.f(GOI_B_INV_MASS, b);
-                    const float ax = gs * gx + im * W.f(GOI_B_FORCE, 2 * b);
-                    const float ay = gs * gy + im * W.f(GOI_B_FORCE, 2 * b + 1);
-                    const float vx = v.x + h * ax, vy = v.y + h * ay;
-                    const float ww = w + h * W.f(GOI_B_INV_INERTIA, b) * W.f(GOI_B_TORQUE, b);
-                    const float ld = 1.0f / (1.0f + h * W.f(GOI_B_LINEAR_DAMPING, b));
-                    const float ad = 1.0f / (1.0f + h * W.f(GOI_B_ANGULAR_DAMPING, b));
-                    v = mk(vx * ld, vy * ld);
-                    w = ww * ad;
-                }
-                W.set2(GOI_B_C0, b, c);
-                W.f(GOI_B_A0, b) = a;
+    for (int b = W.sub; b < W.B; b += W.G) {
+        V2 v = W.v2(GOI_B_V, b);
+        float w = W.f(GOI_B_W, b);
+        const V2 c = W.v2(GOI_B_C, b);
+        const float a = W.f(GOI_B_A, b);
+        if (I.body_island(b) >= 0) {
+            if (W.is_dynamic(b)) {
+                const float gs = W.f(GOI_B_GRAVITY_SCALE, b), im = W.f(GOI_B_INV_MASS, b);
+                const float ax = gs * gx + im * W.f(GOI_B_FORCE, 2 * b);
+                const float ay = gs * gy + im * W.f(GOI_B_FORCE, 2 * b + 1);
+                const float vx = v.x + h * ax, vy = v.y + h * ay;
+                const float ww = w + h * W.f(GOI_B_INV_INERTIA, b) * W.f(GOI_B_TORQUE, b);
+                const float ld = 1.0f / (1.0f + h * W.f(GOI_B_LINEAR_DAMPING, b));
+                const float ad = 1.0f / (1.0f + h * W.f(GOI_B_ANGULAR_DAMPING, b));
+                v = mk(vx * ld, vy * ld);
+                w = ww * ad;
             }
-            bd.set_v(b, v, w);
-            bd.set_c(b, c, a);
-            const Rot q = rot_of(a);
-            bd.at(6, b) = q.c;
-            bd.at(7, b) = q.s;
+            W.set2(GOI_B_C0, b, c);
+            W.f(GOI_B_A0, b) = a;
         }
-        group_sync();
-        if (lanes) {
-            lanes = solve_velocities(m, W, bd, I, s, dt, dt_ratio, lc, lj);
-            if (lanes) break;
-            group_sync();
-            continue;
-        }
-        // the constraint rows are independent of each other: the world's lane group prepares them together (one row
-        // per lane), then every lane solves them in order
-        for (int i = W.sub; i < I.nc; i += W.G) {
-            const int slot = I.corder(i);
-            const int ia = W.ba(slot), ib = W.bb(slot);
-            Rot qA, qB;
-            qA.c = bd.at(6, ia); qA.s = bd.at(7, ia);
-            qB.c = bd.at(6, ib); qB.s = bd.at(7, ib);
-            cs_prepare(m, W, bd, CR, i, slot, warm, dt_ratio, qA, qB, s.velocity_threshold);
-        }
-        for (int i = W.sub; i < I.nj; i += W.G) {
-            const int jid = I.jorder(i);
-            const int ia = m.joint[jid].a, ib = m.joint[jid].b;
-            Rot qA, qB;
-            qA.c = bd.at(6, ia); qA.s = bd.at(7, ia);
-            qB.c = bd.at(6, ib); qB.s = bd.at(7, ib);
-            jn_prepare(m, W, bd, JRw, i, jid, s, dt, dt_ratio, warm, qA, qB);
-        }
-        group_sync();  // rows written by one lane of the group are read by all
-        if (warm)
-            for (int i = 0; i < I.nc; ++i) warm_vrow(bd, load_vrow(CR, i));
-        for (int i = 0; i < I.nj; ++i) jn_warm_start(bd, JRw, i, v24, m.rev_only);
-        for (int it = 0; it < s.velocity_iterations; ++it) {
-            for (int i = 0; i < I.nj; ++i) jn_solve_velocity(bd, JRw, i, v24, m.rev_only);
-            cs_solve_velocity_sweep(bd, CR, 0, I.nc);
-        }
-        // StoreImpulses (contact_solver.py:293-304), rows split over the lane group
-        for (int i = W.sub; i < I.nc; i += W.G) {
-            const int slot = CR.geti(i, CF_SLOT), cnt = CR.geti(i, CF_COUNT);
-            if (cnt > 0) {
-                W.f(GOI_C_NORMAL_IMPULSE, 2 * slot) = CR.getf(i, CF_NI0);
-                W.f(GOI_C_TANGENT_IMPULSE, 2 * slot) = CR.getf(i, CF_TI0);
-            }
-            if (cnt > 1) {
-                W.f(GOI_C_NORMAL_IMPULSE, 2 * slot + 1) = CR.getf(i, CF_NI1);
-                W.f(GOI_C_TANGENT_IMPULSE, 2 * slot + 1) = CR.getf(i, CF_TI1);
-            }
-        }
-        for (int i = W.sub; i < I.nj; i += W.G) jn_store(W, JRw, i, v24);
-        break;
+        bd.set_v(b, v, w);
+        bd.set_c(b, c, a);
+        const Rot q = rot_of(a);
+        bd.at(6, b) = q.c;
+        bd.at(7, b) = q.s;
     }
     group_sync();
-    // integrate positions with the per-step clamps (step.py:120-135)
+}
+
+// integrate positions with the per-step clamps (step.py:120-135)
+GOI_D void integrate_positions(const World& W, const Bodies& bd, const Islands& I, const GoiSettings& s, float h) {
     const float max_t = s.clamps_per_second ? s.max_translation * h : s.max_translation;
     const float max_r = s.clamps_per_second ? s.max_rotation * h : s.max_rotation;
     for (int b = W.sub; b < W.B; b += W.G) {
@@ -306,9 +358,16 @@ GOI_D void solve_world(const DModel& m, const World& W, const Bodies& bd, const 
         bd.set_v(b, v, w);
     }
     group_sync();
-    // position iterations with per-island early exit (step.py:197-251)
-    unsigned long long done = 0ull, all = I.n >= 64 ? ~0ull : ((1ull << I.n) - 1ull);
-    if (lanes && !solve_positions(m, W, bd, CR, JRw, I, s, lc, lj, all, done)) {
+}
+
+// The rows set up in the row tiles, velocity phase, StoreImpulses and positions integrated (all but kPositions), then the
+// position phase (`done`: the islands within tolerance). False when a phase must run again, `how` then says what is left.
+GOI_D bool solve_on_tiles(const DModel& m, const World& W, const Bodies& bd, const Rows& CR, const Rows& JRw,
+                          const Islands& I, const GoiSettings& s, float dt, float dt_ratio, Solve& how,
+                          unsigned long long& done) {
+    const bool warm = s.warm_starting != 0;
+    const float h = dt;
+    if (how == kPositions) {
         // from the integrated poses again (a static body's, outside the islands, may have been written too)
         for (int b = W.sub; b < W.B; b += W.G) {
             const V2 c = W.v2(GOI_B_C, b);
@@ -317,28 +376,81 @@ GOI_D void solve_world(const DModel& m, const World& W, const Bodies& bd, const 
             else bd.set_c(b, c, a);
         }
         group_sync();
-        done = 0ull;
-        lanes = false;
+    } else {
+        // the constraint rows are independent of each other: the world's lane group prepares them together (one row
+        // per lane), then each lane solves its islands' or every lane all of them in order
+        for (int i = W.sub; i < I.nc; i += W.G) {
+            const int slot = I.corder(i);
+            const int ia = W.ba(slot), ib = W.bb(slot);
+            Rot qA, qB;
+            qA.c = bd.at(6, ia); qA.s = bd.at(7, ia);
+            qB.c = bd.at(6, ib); qB.s = bd.at(7, ib);
+            cs_prepare(m, W, bd, CR, i, slot, warm, dt_ratio, qA, qB, s.velocity_threshold);
+        }
+        for (int i = W.sub; i < I.nj; i += W.G) {
+            const int jid = I.jorder(i);
+            const int ia = m.joint[jid].a, ib = m.joint[jid].b;
+            Rot qA, qB;
+            qA.c = bd.at(6, ia); qA.s = bd.at(7, ia);
+            qB.c = bd.at(6, ib); qB.s = bd.at(7, ib);
+            jn_prepare(m, W, bd, JRw, i, jid, s, dt, dt_ratio, warm, qA, qB);
+        }
+        group_sync();  // rows written by one lane of the group are read by all
+        if (!tile_velocities(m, W, bd, CR, JRw, I, s, how == kIslands) && how == kIslands) {
+            how = kRows;
+            return false;
+        }
+        // StoreImpulses (contact_solver.py:293-304), rows split over the lane group
+        for (int i = W.sub; i < I.nc; i += W.G) {
+            const int slot = CR.geti(i, CF_SLOT), cnt = CR.geti(i, CF_COUNT);
+            if (cnt > 0) {
+                W.f(GOI_C_NORMAL_IMPULSE, 2 * slot) = CR.getf(i, CF_NI0);
+                W.f(GOI_C_TANGENT_IMPULSE, 2 * slot) = CR.getf(i, CF_TI0);
+            }
+            if (cnt > 1) {
+                W.f(GOI_C_NORMAL_IMPULSE, 2 * slot + 1) = CR.getf(i, CF_NI1);
+                W.f(GOI_C_TANGENT_IMPULSE, 2 * slot + 1) = CR.getf(i, CF_TI1);
+            }
+        }
+        for (int i = W.sub; i < I.nj; i += W.G) jn_store(W, JRw, i, s.revolute_v24 != 0);
+        group_sync();
+        integrate_positions(W, bd, I, s, h);
     }
-    RotMemo qa, qb;
-    for (int it = 0; !lanes && it < s.position_iterations && done != all; ++it) {
-        unsigned long long jbad = 0ull;
-        for (int i = 0; i < I.n; ++i) W.fwork(i) = 0.0f;  // min separation per island
-        for (int i = 0; i < I.nc; ++i) {
-            const int isl = I.contact_island(I.corder(i));
-            if ((done >> isl) & 1ull) continue;
-            const PRow r = load_prow(CR, i);
-            W.fwork(isl) = bmin(W.fwork(isl), solve_prow(bd, r, s.baumgarte, r.mA, r.mB, r.iA, r.iB, s.linear_slop,
-                                                         s.max_linear_correction, qa, qb));
+    bool ok;
+    done = tile_positions(m, W, bd, CR, JRw, I, s, how == kIslands, ok);
+    if (ok || how != kIslands) return true;
+    how = kPositions;
+    return false;
+}
+
+GOI_D void solve_world(const DModel& m, const World& W, const Bodies& bd, const Rows& CR, const Rows& JRw,
+                            const GoiSettings& s, float dt, const GoiDebug& dbg) {
+    const float dt_ratio = W.f(GOI_S_INV_DT0, 0) * dt;
+    Islands I{W, 0, 0, 0};
+    find_islands(m, W, I);
+    const float h = dt;
+    unsigned long long done = 0ull, all = I.n >= 64 ? ~0ull : ((1ull << I.n) - 1ull);
+    Solve how = rows_fit(m, W, I, s) ? kLanes : m.island_lanes && I.n > 1 ? kIslands : kRows;
+    // The lanes' code first and whole, the tiles' after it, so that the rows in registers are not held across the tiles'
+    // code (a wave's worlds may take both; interleaved by phase, the two spilled 51 to 75 registers, so 0 to 6).
+    integrate_velocities(W, bd, I, h);
+    if (how == kLanes) {
+        LaneContacts lc;
+        LaneJoints lj;
+        if (!solve_velocities(m, W, bd, I, s, dt, dt_ratio, lc, lj)) {
+            group_sync();
+            how = kRows;
+        } else {
+            group_sync();
+            integrate_positions(W, bd, I, s, h);
+            how = solve_positions(m, W, bd, CR, JRw, I, s, lc, lj, all, done) ? kSolved : kPositions;
         }
-        for (int i = 0; i < I.nj; ++i) {
-            const int isl = I.joint_island(JRw.geti(i, JF_JID));
-            if ((done >> isl) & 1ull) continue;
-            if (!jn_solve_position(bd, JRw, i, s, m.rev_only)) jbad |= 1ull << isl;
-        }
-        const float okay_sep = -3.0f * s.linear_slop;
-        for (int i = 0; i < I.n; ++i)
-            if (!((done >> i) & 1ull) && W.fwork(i) >= okay_sep && !((jbad >> i) & 1ull)) done |= 1ull << i;
+        if (how == kRows) integrate_velocities(W, bd, I, h);
+    }
+    while (how != kSolved) {
+        if (solve_on_tiles(m, W, bd, CR, JRw, I, s, dt, dt_ratio, how, done)) break;
+        group_sync();
+        if (how == kRows) integrate_velocities(W, bd, I, h);
     }
     // write back + SynchronizeTransform
     for (int b = W.sub; b < W.B; b += W.G) {

@@ -10,9 +10,10 @@ namespace {
 // What bounds the step is its count of instructions on a world's serial path, so the constants count: with S known,
 // every workspace index is a shift, the lane groups (64 / S lanes) and their exchanges unroll, and no debug code is
 // carried (launches with debug arrays take k_step). kPlain as in k_step_fixed: revolute joints under the v2.4.1 solver
-// and no edge shapes. The dimensions stay run-time values and the State any layout. k_step holds all of this in
-// registers at once and spilled 105 of them (384 B of scratch a lane); these instances spill at most 1 at 1 world a wave
-// and 24 to 35 at 8 (Solve's rows are in registers). When they were added, the 4-body rig with 41 slots (no fixed
+// and no edge shapes. The dimensions stay run-time values and the State any layout. By the compiler's report the instances
+// spill at most 4 vector registers (16 to 32 B of scratch a lane) and 426 to 555 scalar ones, whose reloads are a
+// v_readlane each (the 71 leaf pointers and the dimensions; the rig's fixed instance spills 202 to 246); k_step spills
+// 121 vector registers (496 B) and 653 scalar ones. When they were added, the 4-body rig with 41 slots (no fixed
 // instance): 16,384 worlds, S = 8: 620 -> 497 us a step; 1,024 worlds, S = 1: 435 -> 311 us; the instance for the rig's
 // exact dimensions took 450 us at 16,384 worlds.
 template <int kS, bool kMulti, bool kPlain>

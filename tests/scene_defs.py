@@ -404,3 +404,52 @@ def build_test_scene(name, iterations=None):
     model, state = d.build(contact_capacity=cap)
     cm = wd.compact_model(model, state)
     return s, cm, wd.compact_state(cm, state)
+
+
+def jointed_islands(kind, count, iterations=(8, 3), **settings):
+    """(settings, compact Model, single-world compact State) of `count` groups of bodies joined within themselves only, side
+    by side on the ground, so that a world holds that many islands with joints: "rigs" (the 4-body rig, revolute),
+    "anchored" (two links hung from the ground body, revolute), "pairs" (two boxes on a prismatic joint) and "mixed" (an
+    anchored group, a pair and a welded pair in turn)."""
+    from dataclasses import replace
+    s = replace(Settings.stock(gravity=(0.0, -9.81), continuous_physics=True), velocity_iterations=iterations[0],
+                position_iterations=iterations[1], **settings)
+    d = wd.WorldDef(s)
+    g = d.add_body(wd.STATIC)
+    for i in range(count + 2):
+        d.add_box(g, (2.0, 0.3), (4.0 * i - 4.0, 0.05 * (i % 3)), friction=0.8)
+    for i in range(count):
+        x = 4.0 * i
+        what = kind if kind != "mixed" else ("anchored", "pairs", "weld")[i % 3]
+        if what == "rigs":
+            b2.scenes.add_rig(d, (x - 1.0, 1.2 + 0.1 * i))
+            continue
+        a = d.add_body(wd.DYNAMIC, (x, 0.8), 0.1 * i, mass=1, inertia=0.1)
+        d.add_box(a, (0.4, 0.2), friction=0.5)
+        b = d.add_body(wd.DYNAMIC, (x + 0.9, 0.9), 0.0, mass=0.5, inertia=0.05)
+        d.add_box(b, (0.2, 0.2), friction=0.5)
+        if what == "anchored":
+            d.add_revolute(g, a, (x, 1.5), (0.0, 0.7))
+            d.add_revolute(a, b, (0.5, 0.0), (-0.4, 0.0), limits=(-0.3, 0.3))
+        elif what == "pairs":
+            d.add_prismatic(a, b, (0.4, 0.0), (-0.2, 0.0), (1, 0), 0.0, limits=(-0.05, 0.25))
+        else:
+            d.add_weld(a, b, (0.5, 0.0), (-0.4, 0.0), -0.1 * i)
+    model, state = d.build(contact_capacity=48)
+    cm = wd.compact_model(model, state)
+    return s, cm, wd.compact_state(cm, state)
+
+
+def with_odd_static(state, case):
+    """A batched State whose static bodies' numbers are such that Solve's rows change them (x - 0 * P): "negzero" their
+    velocities -0, "negpose" their poses -0, "nan" a NaN velocity of body 2 in every seventh world; in place."""
+    static = np.asarray(state.bodies.type) == wd.STATIC
+    names = {"negzero": ("v", "w"), "negpose": ("c", "a")}.get(case, ())
+    for name in names:
+        leaf = getattr(state.bodies, name)
+        zero = (static if leaf.ndim == 2 else static[..., None]) & (leaf == 0.0)
+        assert zero.any()
+        leaf[...] = np.where(zero, F32(-0.0), leaf)
+    if case == "nan":
+        state.bodies.v[1::7, 2, 1] = np.nan
+    return state

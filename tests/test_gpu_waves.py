@@ -105,3 +105,46 @@ def test_search_on_lane_groups(oracle, monkeypatch, scene, slots, wpw):
         assert bad == [], f"step {k + 1}: {bad[:4]}"
     live = (np.asarray(ref.contacts.pair) >= 0).sum(1)
     assert live.max() == slots if slots in (3, 20) else live.max() > 4
+
+
+@pytest.mark.parametrize("wpw", [1, 2, 4, 8])
+@pytest.mark.parametrize("kind,count", [("rigs", 6), ("anchored", 8), ("pairs", 8), ("mixed", 9)])
+def test_jointed_islands(oracle, monkeypatch, kind, count, wpw):
+    """Several islands with joints of their own: revolute rows in registers, islands side by side in levels (1 and 2 worlds
+    a wave; more rows than lanes at 4 and 8), and row tiles with an island a lane (other joints, the v2.3.1 solver, too
+    many rows). Then static bodies with -0 velocities or poses, and a NaN, where the rows must run one after another."""
+    from dataclasses import replace
+    monkeypatch.setenv("GOI_WORLDS_PER_WAVE", str(wpw))
+    s, m, one = scene_defs.jointed_islands(kind, count)
+    ref = perturbed(one, 29)
+    for settings in (s, replace(s, revolute_v24=False)):
+        ref = _compare(m, ref, settings, 0.02, 12, oracle)
+        ref = _compare(m, ref, settings, 0.02, 2, oracle, n_steps=3)
+        assert b2.last_launch()["worlds_per_wave"] == wpw
+        assert int(np.asarray(ref.contacts.touching).sum(1).max()) >= 2
+        for case in ("negzero", "negpose", "nan"):
+            _compare(m, scene_defs.with_odd_static(oracle.copy(ref), case), settings, 0.02, 4, oracle, nan_equal=True)
+
+
+@pytest.mark.parametrize("kind,n,v24", [("pairs", 256, True), ("rigs", 256, True), ("rigs", 256, False)])
+def test_islands_do_not_add_up(kind, n, v24):
+    """A world's islands are solved side by side, whatever their joints: six of them in a world take less than half of six
+    times one (one after another they took most of it, at 300 / 30 iterations, where Solve is the step)."""
+    def step_us(count):
+        s, m, one = scene_defs.jointed_islands(kind, count, iterations=(300, 30), revolute_v24=v24)
+        dev = b2.layout.to_device(perturbed(one, n), "cuda")
+        for _ in range(8):
+            b2.step_(m, dev, s, 0.02)
+        times = []
+        for _ in range(5):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(4):
+                b2.step_(m, dev, s, 0.02)
+            end.record()
+            end.synchronize()
+            times.append(start.elapsed_time(end) / 4 * 1000)
+        return min(times)
+    one, six = step_us(1), step_us(6)
+    print(f"one island {one:.0f} us a step, six {six:.0f}")
+    assert six < 3 * one, f"one island {one:.0f} us a step, six {six:.0f}"

@@ -198,6 +198,24 @@ def test_nonfinite_islands_sanitized(host_step, tmp_path, oracle):
         check(run(host_step, p, "step"))
 
 
+@pytest.mark.parametrize("v24", [True, False])
+@pytest.mark.parametrize("kind,count", [("rigs", 2), ("rigs", 6), ("anchored", 4), ("pairs", 8), ("mixed", 9)])
+def test_jointed_islands_sanitized(host_step, tmp_path, oracle, kind, count, v24):
+    """Several islands with joints of their own: revolute rows in registers (up to 8 joints on the host's one lane) or the
+    islands one by one from the row tiles; then static bodies with -0 velocities or poses, and a NaN."""
+    from dataclasses import replace
+    s, m, one = scene_defs.jointed_islands(kind, count)
+    s, st = replace(s, revolute_v24=v24), perturbed(one, 8)
+    p = tmp_path / "scn.bin"
+    write_scenario(p, m, st, s, 0.02, 25, False)
+    check(run(host_step, p, "step"))
+    for _ in range(15):
+        oracle.step_(m, st, s, np.float32(0.02))
+    for case in ("negzero", "negpose", "nan"):
+        write_scenario(p, m, scene_defs.with_odd_static(oracle.copy(st), case), s, 0.02, 6, False)
+        check(run(host_step, p, "step"))
+
+
 @pytest.mark.parametrize("dt", [0.0, -0.02])
 def test_non_positive_dt_sanitized(host_step, tmp_path, dt):
     """dt <= 0: Solve still runs (step.py:35-40) and SolveTOI is skipped (toi.py:841); inv_dt0 keeps its value."""
