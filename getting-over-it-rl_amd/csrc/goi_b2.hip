@@ -683,6 +683,13 @@ static long blocks_per_cu(size_t lds) {
 // large. The 4-body rig with 40 slots: 8 worlds per wave, 8 blocks per CU. The rig with 12 boxes and 128 slots: 4
 // worlds per wave (30.6 KB, 5 blocks per CU: 20 worlds) rather than 8 (61 KB, 2 blocks: 16 worlds), measured 35%
 // faster at 65536 worlds.
+//
+// The choice ends at 8, the largest size with an instance of its own, also where a CU would hold more worlds at 16 or 32
+// (few slots): k_step takes those, a world there has 2 or 4 lanes, and blocks of 8 in rounds do not wait for each other.
+// us a step at 8 / 16 a wave: the rig with 12 slots, 17,000 worlds 335 / 751, 65,536 worlds 837 / 900; with 30 slots
+// 326 / 600 and 886 / 1320; 4 loose boxes on the terrain at 25 m/s, 12 slots, 17,000 worlds 1849 / 2446. Only worlds with
+// next to nothing to solve are faster at 16 (20,000 stacks of boxes 139 / 92, 65,536 balls on a plank 145 / 119).
+constexpr int kMaxAutoWave = kBlock < 8 ? kBlock : 8;
 static int worlds_per_wave(int n, size_t ws_bytes_per_world) {
     const char* e = getenv("GOI_WORLDS_PER_WAVE");  // read per call: tests vary it within one process
     int forced = e ? atoi(e) : 0;
@@ -691,7 +698,7 @@ static int worlds_per_wave(int n, size_t ws_bytes_per_world) {
         return std::min<long>(forced, std::max<long>(1, (kMaxLdsBytes - kBlock * sizeof(int)) / ws_bytes_per_world));
     int wpw = 0;
     long best = -1;
-    for (int w = 1; w <= kBlock; w *= 2) {
+    for (int w = 1; w <= kMaxAutoWave; w *= 2) {
         const size_t lds = ws_bytes_per_world * w + kBlock * sizeof(int);
         if (lds > kMaxLdsBytes) break;
         const long blocks = blocks_per_cu(lds);
@@ -797,8 +804,8 @@ static int check_step_args(const GoiModel* model, const GoiStateView* state, con
     return GOI_OK;
 }
 
-// The step instance compiled for wpw worlds per wave, or null: k_step takes the other wave sizes (a forced odd one; 16
-// and above, for worlds with so few slots that a CU's LDS holds more of them that way) and launches with debug arrays.
+// The step instance compiled for wpw worlds per wave, or null: k_step takes the other wave sizes (forced ones only)
+// and launches with debug arrays.
 using WaveLaunch = hipError_t (*)(const DModel&, const Launch&, bool, bool, dim3, size_t, hipStream_t);
 static WaveLaunch wave_instance(int wpw) {
 #ifdef GOI_HOST_BUILD

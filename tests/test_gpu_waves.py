@@ -48,11 +48,13 @@ def test_wave_instances_parity(oracle, monkeypatch, case, wpw):
         assert b2.last_launch()["worlds_per_wave"] == wpw
 
 
-@pytest.mark.parametrize("n", [1, 2047, 2048, 2049, 4097, 8193, 16383, 16384, 16385])
-def test_wave_size_rule(oracle, n):
+@pytest.mark.parametrize("n,slots", [(1, 40), (2047, 40), (2048, 40), (2049, 40), (4097, 40), (8193, 40), (16383, 40),
+                                     (16384, 40), (16385, 40), (16384, 24), (16385, 24), (20000, 8), (40000, 12)])
+def test_wave_size_rule(oracle, n, slots):
     """The smallest wave size whose blocks all fit the GPU at once (8 blocks a CU for the rig), the most resident one
-    above that; two steps at the edges of each range."""
-    s, m, st, cfg = b2.scenes.make_config(4, min(n, 256))
+    above that, up to 8 (a CU holds more rig worlds of 24 slots or fewer at 16 or 32 a wave); two steps at the edges of
+    each range."""
+    s, m, st, cfg = b2.scenes.make_config(4, min(n, 256), capacity=slots)
     idx = np.arange(n) % min(n, 256)
     st = b2.world.from_leaves([np.ascontiguousarray(x[idx]) for x in b2.world.leaves(st)])
     _compare(m, st, s, cfg.dt, 2, oracle)
