@@ -5,8 +5,9 @@
 // the run at its source line, which a fault on the device does not give.
 //
 // Usage: host_step <scenario file> <mode> [plant], mode "step" (goi_step), "step_n:K" (goi_step_n, K steps a
-// launch) or "noalloc:K" (goi_step_n_noalloc); "plant" moves the last world's first body by one ulp in the oracle's
-// copy only, so that run must end in a mismatch. The scenario file (written by tests/test_host_sanitized.py,
+// launch) or "noalloc:K" (goi_step_n_noalloc), each with ":debug" after it to pass every GoiDebug array (which takes the
+// general k_step) and compare those with the oracle's too; "plant" moves the last world's first body by one ulp in the
+// oracle's copy only, so that run must end in a mismatch. The scenario file (written by tests/test_host_sanitized.py,
 // little-endian):
 //   "GOISCN02", int32 F J P B, then the 24 GoiModelDesc arrays in declaration order, each an int64 byte count
 //   (-1 = NULL) and the bytes; int32 sizeof(GoiSettings) and the struct; float dt; int32 n_steps, n, B R J C,
@@ -76,7 +77,10 @@ struct Leaf {
 int main(int argc, char** argv) {
     if (argc != 3 && !(argc == 4 && std::strcmp(argv[3], "plant") == 0))
         die("usage: host_step <scenario> <step | step_n:K | noalloc:K> [plant]");
-    const std::string mode = argv[2];
+    std::string mode = argv[2];
+    const size_t at = mode.rfind(":debug");
+    const bool debug = at != std::string::npos && at + 6 == mode.size();
+    if (debug) mode.resize(at);
     const bool plant = argc == 4;  // nudge the oracle's input by one ulp: the run must then report a mismatch
     int per_launch = 1;
     bool noalloc = false, step_n = false;
@@ -201,6 +205,27 @@ int main(int argc, char** argv) {
         ref_leaves[l] = leaves[l].ref;
     }
 
+    // the debug arrays of both sides, [rows][pitch] (one per field of GoiDebug in its order), and the oracle's batch is n
+    // worlds wide: the library's pitch must be n
+    if (debug && pitch != n) die("debug arrays need one buffer per leaf");
+    const size_t traced = GOI_DEBUG_TOI_EVENTS;
+    const char* const dbg_names[9] = {"body_island", "contact_island", "contact_order", "n_islands", "toi_event_slot",
+                                      "toi_event_alpha", "toi_event_island", "toi_island_rows", "status"};
+    const size_t dbg_rows[9] = {(size_t)B, (size_t)C, (size_t)C, 1, traced, traced, traced,
+                                traced * GOI_DEBUG_TOI_ROWS, 1};
+    int32_t *dbg_lib[9] = {}, *dbg_ref[9] = {};
+    for (int f = 0; debug && f < 9; ++f) {
+        dbg_lib[f] = (int32_t*)block(dbg_rows[f] * n * 4);
+        dbg_ref[f] = (int32_t*)block(dbg_rows[f] * n * 4);
+    }
+    const auto dbg_of = [](int32_t* const* a) {
+        return GoiDebug{a[0], a[1], a[2], a[3], a[4], a[5], a[6], a[7], a[8]};
+    };
+    const GoiDebug lib_dbg = dbg_of(dbg_lib);
+    GoiDebug ref_dbg = dbg_of(dbg_ref);
+    const GoiDebug* const lib_arg = debug ? &lib_dbg : nullptr;
+    GoiDebug* const ref_arg = debug ? &ref_dbg : nullptr;
+
     long compared = 0;
     for (int k0 = 0; k0 < n_steps; k0 += per_launch) {
         const int k1 = std::min(n_steps, k0 + per_launch);
@@ -219,16 +244,29 @@ int main(int argc, char** argv) {
                 tq[(size_t)w * J + motor] = torque_gain * std::sqrt(ax * ax + ay * ay);
             }
         }
+        for (int f = 0; debug && f < 9; ++f) {  // filled apart: an entry that either side leaves shows
+            std::memset(dbg_lib[f], 0x5a, dbg_rows[f] * n * 4);
+            std::memset(dbg_ref[f], 0xa5, dbg_rows[f] * n * 4);
+        }
         int rc;
         if (noalloc)
-            rc = goi_step_n_noalloc(model, &view, &s, dt, k1 - k0, nullptr, nullptr);
+            rc = goi_step_n_noalloc(model, &view, &s, dt, k1 - k0, nullptr, lib_arg);
         else if (step_n)
-            rc = goi_step_n(model, &view, &s, dt, k1 - k0, nullptr, nullptr);
+            rc = goi_step_n(model, &view, &s, dt, k1 - k0, nullptr, lib_arg);
         else
-            rc = goi_step(model, &view, &s, dt, nullptr, nullptr);
+            rc = goi_step(model, &view, &s, dt, nullptr, lib_arg);
         if (rc != GOI_OK) die(std::string("step: ") + goi_last_error());
         for (int k = k0; k < k1; ++k)
-            if (oracle_step(&d, ref_leaves.data(), n, B, C, R, J, &s, dt, 1, nullptr) != 0) die("oracle_step failed");
+            if (oracle_step(&d, ref_leaves.data(), n, B, C, R, J, &s, dt, 1, ref_arg) != 0) die("oracle_step failed");
+        for (int f = 0; debug && f < 9; ++f)
+            for (size_t i = 0; i < dbg_rows[f] * n; ++i, ++compared)
+                if (dbg_lib[f][i] != dbg_ref[f][i]) {
+                    std::printf("MISMATCH after step %d: debug array %s row %zu world %zu (oracle 0x%08x, step 0x%08x)\n",
+                                k1, dbg_names[f], i / n, i % n, dbg_ref[f][i], dbg_lib[f][i]);
+                    std::fflush(stdout);
+                    goi_model_destroy(model);
+                    return 1;
+                }
         for (const Leaf& L : leaves)
             for (int w = 0; w < n; ++w)
                 for (int64_t i = 0; i < L.per_world; ++i) {

@@ -48,8 +48,8 @@ def test_scene_parity(name, oracle):
 @pytest.mark.parametrize("name,wpw", [("pile", 2), ("pile", 8), ("joints", 16), ("polygons", 16), ("misc", 8)])
 def test_islands_side_by_side_parity(name, wpw, oracle, monkeypatch):
     """Scenes of several islands (pile up to 12, polygons 9, joints 8 with every joint type, misc 6) at wave shapes
-    whose lane groups hold fewer lanes than the world has islands (2 to 32 lanes), so lanes take several islands
-    each: 64 perturbed copies, 60 steps."""
+    whose lane groups hold fewer lanes than the world has islands (2 to 32 lanes), so lanes take several rows,
+    or (other joints than revolute) several islands, each: 64 perturbed copies, 60 steps."""
     monkeypatch.setenv("GOI_WORLDS_PER_WAVE", str(wpw))
     s, m, st = scene_defs.build_test_scene(name, iterations=(8, 3))
 
@@ -269,7 +269,7 @@ def test_toi_event_traces(oracle):
 @pytest.mark.parametrize("n_steps", [1, 4])
 def test_packed_and_unpacked_states_agree(n_steps, monkeypatch):
     """The 4-body rig on a packed State (one buffer, every leaf at its packed offset: the fixed-dimension kernel of
-    goi_b2_rig.hip) and on the same State with one buffer per leaf (the general kernel) step to identical States, for
+    goi_b2_rig.hip) and on the same State with one buffer per leaf (the instance for 8 worlds a wave) step to identical States, for
     single steps and for goi_step_n."""
     monkeypatch.setenv("GOI_WORLDS_PER_WAVE", "8")  # the rig kernel's 8 worlds per wave at this batch size
     s, m, st, cfg = b2.scenes.make_config(4, 512)
@@ -423,8 +423,8 @@ def test_step_n_equals_repeated_steps(oracle, monkeypatch, case, wpw, k):
 def test_multi_round_launches(oracle, monkeypatch, case):
     """Launches with more blocks than the GPU holds at once run their blocks in the order k_group_order gives (the
     world groups with the most TOI events of the previous step first): config 5 at 8,192 worlds (2,048 blocks of the
-    island instance, 5 a CU) and config 4 at 16,384 worlds with 4 worlds a wave (4,096 blocks of the generic kernel,
-    8 a CU). 6 steps with actions, bit for bit."""
+    island instance, 5 a CU) and config 4 at 16,384 worlds with 4 worlds a wave (4,096 blocks of the
+    instance for any dimensions, 8 a CU). 6 steps with actions, bit for bit."""
     if case == "island":
         monkeypatch.setenv("GOI_WORLDS_PER_WAVE", "4")
         s, m, st, cfg = b2.scenes.make_config(5, 8192, edges="quad")
@@ -445,8 +445,8 @@ def test_multi_round_launches(oracle, monkeypatch, case):
 @pytest.mark.parametrize("case", ["island", "native_edges"])
 def test_other_kernels_with_lanes_without_a_world(oracle, monkeypatch, case):
     """A partly filled last block on the island instance (config 5, 250 worlds at 4 a wave on a packed State of pitch
-    256: its SolveTOI re-derives its views in each event iteration) and on the generic kernel with native edge shapes
-    (config 4 with a b2ChainShape terrain, 250 worlds at 8 a wave). 8 steps with actions, bit for bit."""
+    256: its SolveTOI re-derives its views in each event iteration) and on the instance for any dimensions with native
+    edge shapes (config 4 with a b2ChainShape terrain, 250 worlds at 8 a wave). 8 steps with actions, bit for bit."""
     if case == "island":
         monkeypatch.setenv("GOI_WORLDS_PER_WAVE", "4")
         s, m, st, cfg = b2.scenes.make_config(5, 250, edges="quad")
@@ -468,7 +468,7 @@ def test_other_kernels_with_lanes_without_a_world(oracle, monkeypatch, case):
 def test_step_n_lanes_without_a_world(oracle, monkeypatch, wpw, n, pitch):
     """step_n_ (3 steps a launch, two launches) on blocks with lanes that run no world: the multi-step path sets up
     each step's cooperative views afresh as the single step does. The rig's multi-step instance on a packed State of
-    pitch 256 with 250 worlds, the generic kernel at 20 and 13 worlds per wave. Config 4 with actions, bit for bit."""
+    pitch 256 with 250 worlds, the general k_step at 20 and 13 worlds per wave. Config 4 with actions, bit for bit."""
     monkeypatch.setenv("GOI_WORLDS_PER_WAVE", str(wpw))
     s, m, st, cfg = b2.scenes.make_config(4, n, capacity=40)
     rng = np.random.default_rng(29)
@@ -513,10 +513,10 @@ def test_island_kernel_parity(oracle, monkeypatch):
 
 @pytest.mark.parametrize("wpw", ["4", "8"])
 def test_nonfinite_islands_parity(oracle, monkeypatch, wpw):
-    """Worlds of several islands, whose lanes solve the islands side by side, with a NaN or infinite value in one
+    """Worlds of several islands, whose lanes solve the islands' rows side by side, with a NaN or infinite value in one
     island (test_host_sanitized.nonfinite_islands_case, 64 worlds): Box2D's order carries it through the terrain into
-    the other islands, which the device must follow by solving those worlds' islands one after another. 20 steps,
-    NaN for NaN, on the island instance (4 worlds per wave) and the general kernel (8)."""
+    the other islands, which the device must follow by solving those worlds' rows one after another. 20 steps,
+    NaN for NaN, on the island instance (4 worlds per wave) and the one for any dimensions (8)."""
     from test_host_sanitized import nonfinite_islands_case
     monkeypatch.setenv("GOI_WORLDS_PER_WAVE", wpw)
     m, st, s, dt = nonfinite_islands_case(oracle, n=64)
@@ -655,8 +655,8 @@ def test_nonfinite_worlds_parity(oracle, monkeypatch, wpw):
     """NaN and infinite values written into a few worlds of config 4 (a NaN velocity, an infinite spin, a NaN
     position, 1e30 m/s, a NaN force; the failure inputs of the reference's bench, bench_gpu.py:135-136): the other
     worlds stay bit-exact and the poisoned ones follow the oracle, NaN for NaN (a box with a NaN coordinate overlaps
-    every box under b2TestOverlap, so their tables fill and overflow). 64 worlds, 30 steps, the general kernel and the
-    rig instance (8 worlds per wave). The same scenario runs first under the sanitizers on the CPU
+    every box under b2TestOverlap, so their tables fill and overflow). 64 worlds, 30 steps, the instance for one world
+    a wave and the rig instance (8). The same scenario runs first under the sanitizers on the CPU
     (test_host_sanitized.py::test_nonfinite_worlds_sanitized)."""
     from test_host_sanitized import nonfinite_case
     if wpw is not None:
@@ -697,7 +697,7 @@ def test_max_events_parity(oracle, monkeypatch, max_events):
 def test_status_word_parity(oracle):
     """GoiDebug.status (the step's failure counters as one word per world) on the device equals the oracle's at every
     step, with every bit raised somewhere: non-finite worlds (which also overflow their tables), max_events 2
-    (SolveTOI capped) and one step of dt 0 (SolveTOI skipped). Config 4, 64 worlds, 12 steps, the general kernel (a
+    (SolveTOI capped) and one step of dt 0 (SolveTOI skipped). Config 4, 64 worlds, 12 steps, the general k_step (a
     launch with debug arrays takes it); the other debug arrays and every leaf are compared too, NaN for NaN."""
     from dataclasses import replace
     from test_host_sanitized import nonfinite_case

@@ -64,11 +64,13 @@ def test_wave_size_rule(oracle, n, slots):
     assert info["worlds_per_wave"] == want and info["blocks"] == -(-n // want), info
 
 
-@pytest.mark.parametrize("wpw,case", [(8, "piles"), (4, "piles"), (8, "negzero"), (1, "negzero"), (2, "nan")])
+@pytest.mark.parametrize("wpw,case", [(8, "piles"), (4, "piles"), (8, "negzero"), (1, "negzero"), (2, "nan"),
+                                      (1, "negpose"), (4, "negpose"), (8, "negpose")])
 def test_solver_rows_beyond_the_lanes(oracle, monkeypatch, wpw, case):
     """Solve's rows in the lanes' registers and the cases that leave them: more touching contacts than a group's lanes
-    hold (piles at 8 worlds a wave: 16 rows; some worlds have more, others fewer), a static body whose velocity is -0
-    (x - 0 * P may turn it into +0, which the other lanes' rows must see), and a NaN that reaches the terrain."""
+    hold (piles at 8 worlds a wave: 16 rows; some worlds have more, others fewer), a static body whose velocity or pose
+    is -0 (x - 0 * P may turn it into +0, which the other lanes' rows must see: the velocity phase runs again, or the
+    position phase on rows written from the registers), and a NaN that reaches the terrain."""
     monkeypatch.setenv("GOI_WORLDS_PER_WAVE", str(wpw))
     s, m, st, cfg = b2.scenes.make_config(5, 48)
     for _ in range(60):
@@ -78,6 +80,8 @@ def test_solver_rows_beyond_the_lanes(oracle, monkeypatch, wpw, case):
     if case == "negzero":
         st.bodies.v[:, 0] = np.float32(-0.0)
         st.bodies.w[:, 0] = np.float32(-0.0)
+    elif case == "negpose":
+        st = scene_defs.with_odd_static(st, case)
     elif case == "nan":
         st.bodies.v[1::7, 9, 1] = np.nan
     _compare(m, st, s, cfg.dt, 6, oracle, nan_equal=True)

@@ -1,14 +1,15 @@
-"""The step's own code on the CPU under AddressSanitizer and UBSan: the library's two translation units compiled for
+"""The step's own code on the CPU under AddressSanitizer and UBSan: the library's translation units compiled for
 the host (GOI_HOST_BUILD: blocks and lanes run one after another, every workspace, row tile and State leaf an
 exactly-sized heap block) step the same worlds as the oracle (also sanitized), and every State leaf is compared bit
 for bit after every launch (tests/host_step). An out-of-bounds access or an undefined operation in the step stops
 the run with its source line; a wrong result shows as a mismatch. This is where a device fault is localised: the
 same code, the same scenario, on the CPU.
 
-Covers the general step (one buffer per leaf), the fixed-dimension rig and island steps (packed States), goi_step_n and
+Covers the step for one world a wave and any State (k_step_waves<1>, one buffer per leaf), the general k_step (launches
+with debug arrays, which are compared too), the fixed-dimension rig and island steps (packed States), goi_step_n and
 goi_step_n_noalloc, the TOI and edge scenes and the island-heavy configuration. The host build runs one world per
-one-lane block, so the lane-group exchanges it checks are those of groups of one lane; the device's wider groups
-are covered by the GPU parity tests."""
+one-lane block, so the lane-group exchanges it checks are those of groups of one lane, and a lane keeps up to 32 contact
+and 8 joint rows in "registers"; the device's wider groups are covered by the GPU parity tests."""
 import fcntl
 import importlib
 import os
@@ -99,6 +100,11 @@ def check(r):
         f"exit {r.returncode}\n{r.stdout[-1500:]}\n{r.stderr[-6000:]}")
 
 
+def kernels(r):
+    """The names of the step kernels a run launched, in order."""
+    return [ln.split()[1] for ln in r.stderr.splitlines() if ln.startswith("launch ") and "k_step" in ln]
+
+
 def config_case(k, n, steps, edges="quad", seed=7):
     s, m, st, cfg = b2.scenes.make_config(k, n, edges=edges)
     rng = np.random.default_rng(seed)
@@ -106,20 +112,41 @@ def config_case(k, n, steps, edges="quad", seed=7):
     return m, st, s, cfg.dt, acts
 
 
-@pytest.mark.parametrize("packed", [True, False], ids=["packed-rig", "per-leaf-general"])
+@pytest.mark.parametrize("packed", [True, False], ids=["packed-rig", "per-leaf-waves"])
 @pytest.mark.parametrize("edges", ["quad", "native"])
 def test_config4_sanitized(host_step, tmp_path, packed, edges):
     """The benchmark rig (config 4) with actions: the packed State takes the fixed-dimension rig kernel, the State
-    with one buffer per leaf the general kernel."""
+    with one buffer per leaf the instance for one world a wave."""
     m, st, s, dt, acts = config_case(4, 256, 60, edges)
     p = tmp_path / "scn.bin"
     write_scenario(p, m, st, s, dt, 60, packed, acts)
     r = run(host_step, p, "step")
     check(r)
     assert "60 steps" in r.stdout
-    launches = [ln for ln in r.stderr.splitlines() if ln.startswith("launch ") and "k_step" in ln]
-    assert len(launches) == 60
-    assert all(("k_step_fixed" in ln) == packed for ln in launches), launches[:2]
+    ran = kernels(r)
+    assert len(ran) == 60
+    assert all(("k_step_fixed<kRig" if packed else "k_step_waves<kS") in k for k in ran), ran[:2]
+
+
+@pytest.mark.parametrize("case,mode", [("rig", "step:debug"), ("native", "step_n:3:debug"), ("piles", "step:debug"),
+                                       ("joints", "step:debug"), ("joints_v23", "noalloc:2:debug")])
+def test_debug_launches_sanitized(host_step, tmp_path, case, mode):
+    """Launches with every debug array take the general k_step; the arrays (islands, solve order, TOI traces, status) and
+    the State equal the oracle's."""
+    acts = None
+    if case in ("rig", "native", "piles"):
+        k, n, steps = (5, 6, 45) if case == "piles" else (4, 32, 30)
+        m, st, s, dt, acts = config_case(k, n, steps, "native" if case == "native" else "quad")
+        acts = acts if mode == "step:debug" else None
+    else:
+        s, m, one = scene_defs.build_test_scene(case, iterations=(8, 3))
+        st, dt, steps = perturbed(one, 12), 1.0 / 60.0, 40
+    p = tmp_path / "scn.bin"
+    write_scenario(p, m, st, s, dt, steps, False, acts)
+    r = run(host_step, p, mode)
+    check(r)
+    ran = kernels(r)
+    assert ran and all(k.startswith(("k_step<", "(k_step<")) for k in ran), ran[:2]
 
 
 @pytest.mark.parametrize("n", [4093, 4500])
@@ -136,14 +163,14 @@ def test_block_order_many_chunks(host_step, tmp_path, n):
 
 @pytest.mark.parametrize("poison", ["8", "-1", "0"])
 def test_poisoned_scratch_sanitized(host_step, tmp_path, poison):
-    """The benchmark rig (packed: the fixed instance) and the general kernel with the LDS workspaces and rows filled
-    with small integers instead of NaN before every launch (8 as a body or slot index, -1 as an empty slot, 0): the
-    same results, so no pass reads a word its launch has not written."""
+    """The benchmark rig (packed: the fixed instance), the instance for one world a wave and the general k_step with the
+    LDS workspaces and rows filled with small integers instead of NaN before every launch (8 as a body or slot index, -1
+    as an empty slot, 0): the same results, so no pass reads a word its launch has not written."""
     m, st, s, dt, acts = config_case(4, 64, 30)
-    for packed in (True, False):
+    for packed, mode in ((True, "step"), (False, "step"), (False, "step:debug")):
         p = tmp_path / f"scn{int(packed)}.bin"
         write_scenario(p, m, st, s, dt, 30, packed, acts)
-        check(run(host_step, p, "step", poison=poison))
+        check(run(host_step, p, mode, poison=poison))
 
 
 def nonfinite_case(n=64, steps=30, seed=7):
@@ -163,21 +190,21 @@ def nonfinite_case(n=64, steps=30, seed=7):
 
 def test_nonfinite_worlds_sanitized(host_step, tmp_path):
     """NaN and infinite body values step without an out-of-bounds access or undefined operation in either the
-    library's step or the oracle, to the same bits (both run here on the same float hardware), on the rig instance
-    and the general kernel."""
+    library's step or the oracle, to the same bits (both run here on the same float hardware), on the rig instance,
+    the instance for one world a wave and the general k_step."""
     m, st, s, dt, acts = nonfinite_case()
-    for packed in (True, False):
+    for packed, mode in ((True, "step"), (False, "step"), (False, "step:debug")):
         p = tmp_path / f"scn{int(packed)}.bin"
         write_scenario(p, m, st, s, dt, 30, packed, acts)
-        check(run(host_step, p, "step"))
+        check(run(host_step, p, mode))
 
 
 def nonfinite_islands_case(oracle, n=8, clean=50):
     """Config 5 after `clean` steps on the oracle (its worlds then hold 1 to 11 awake islands), with non-finite values
     written into one island of a few worlds: a NaN linear velocity of a box (world 1), an infinite angular velocity
     (world 3) and a NaN force (world 5). In Box2D's order a non-finite impulse reaches the terrain's velocity
-    (v - 0 * P) and from there the world's other islands; the library, whose lanes solve a world's islands side by
-    side, must then solve that world's islands one after another to give the same bits."""
+    (v - 0 * P) and from there the world's other islands; the library, whose lanes solve a world's rows side by
+    side where they share no moving body, must then solve that world's rows one after another to give the same bits."""
     s, m, st, cfg = b2.scenes.make_config(5, n)
     for _ in range(clean):
         oracle.step_(m, st, s, cfg.dt)
@@ -190,11 +217,25 @@ def nonfinite_islands_case(oracle, n=8, clean=50):
 
 def test_nonfinite_islands_sanitized(host_step, tmp_path, oracle):
     """Worlds of several islands with non-finite values in one of them step to the oracle's bits, on the island
-    instance and the general kernel."""
+    instance, the instance for one world a wave and the general k_step."""
     m, st, s, dt = nonfinite_islands_case(oracle)
-    for packed in (True, False):
+    for packed, mode in ((True, "step"), (False, "step"), (False, "step:debug")):
         p = tmp_path / f"scn{int(packed)}.bin"
         write_scenario(p, m, st, s, dt, 20, packed)
+        check(run(host_step, p, mode))
+
+
+@pytest.mark.parametrize("k,case", [(4, "negpose"), (5, "negpose"), (5, "negzero")])
+def test_static_negative_zero_sanitized(host_step, tmp_path, oracle, k, case):
+    """A terrain body whose pose or velocity is -0 (x - 0 * P may turn it into +0, which the rows after it see): the
+    velocity or the position phase runs again row after row, on the fixed instances and the one for any State."""
+    s, m, st, cfg = b2.scenes.make_config(k, 16)
+    for _ in range(40 if k == 5 else 10):
+        oracle.step_(m, st, s, cfg.dt)
+    st = scene_defs.with_odd_static(st, case)
+    for packed in (True, False):
+        p = tmp_path / f"scn{int(packed)}.bin"
+        write_scenario(p, m, st, s, cfg.dt, 8, packed)
         check(run(host_step, p, "step"))
 
 
@@ -240,7 +281,7 @@ def test_max_events_sanitized(host_step, tmp_path, max_events):
 @pytest.mark.parametrize("capacity", [6, 10])
 def test_contact_table_overflow_sanitized(host_step, tmp_path, capacity):
     """Config 4 with 6 or 10 contact slots a world: FindNewContacts drops pairs (overflow > 0 in many worlds) and
-    those worlds keep full candidate searches; the general kernel (the fixed rig instance needs 40 slots)."""
+    those worlds keep full candidate searches; the instance for any State (the fixed rig instance needs 40 slots)."""
     s, m, st, cfg = b2.scenes.make_config(4, 64, capacity=capacity)
     rng = np.random.default_rng(31)
     acts = np.stack([b2.scenes.actions(rng, 64) for _ in range(40)])
@@ -260,17 +301,17 @@ def test_multi_step_launches_sanitized(host_step, tmp_path, mode):
     check(run(host_step, p, mode))
 
 
-@pytest.mark.parametrize("packed", [True, False], ids=["packed-island", "per-leaf-general"])
+@pytest.mark.parametrize("packed", [True, False], ids=["packed-island", "per-leaf-waves"])
 def test_config5_sanitized(host_step, tmp_path, packed):
     """Config 5's box piles: 128 contact slots a world, large islands. The packed State takes the instance compiled
-    for these dimensions, one buffer per leaf the general kernel."""
+    for these dimensions, one buffer per leaf the instance for one world a wave."""
     m, st, s, dt, _ = config_case(5, 8, 60)
     p = tmp_path / "scn.bin"
     write_scenario(p, m, st, s, dt, 60, packed)
     r = run(host_step, p, "step")
     check(r)
-    launches = [ln for ln in r.stderr.splitlines() if ln.startswith("launch ") and "k_step" in ln]
-    assert len(launches) == 60 and all(("k_step_fixed<kIsland" in ln) == packed for ln in launches), launches[:2]
+    ran = kernels(r)
+    assert len(ran) == 60 and all(("k_step_fixed<kIsland" if packed else "k_step_waves<kS") in k for k in ran), ran[:2]
 
 
 @pytest.mark.parametrize("name", ["pile", "joints", "joints_v23", "misc", "hammer_chain", "multi_event",
@@ -324,5 +365,5 @@ def test_full_layout_state_sanitized(host_step, tmp_path, case):
     write_scenario(p, m, st, s, dt, steps, True, acts)
     r = run(host_step, p, "step")
     check(r)
-    launches = [ln for ln in r.stderr.splitlines() if ln.startswith("launch ") and "k_step" in ln]
-    assert launches and not any("k_step_fixed" in ln for ln in launches)
+    ran = kernels(r)
+    assert ran and all("k_step_waves<kS" in k for k in ran), ran[:2]

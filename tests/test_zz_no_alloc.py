@@ -33,7 +33,7 @@ def _call(fn, m, dev, s, dt, n_steps):
 
 @pytest.mark.parametrize("wpw,kernel", [(None, "generic"), ("8", "rig")])
 def test_noalloc_equals_step_n_twice(monkeypatch, wpw, kernel):
-    """The default wave size (1 world a wave at these batch sizes: the generic kernel) and 8 worlds a wave (the
+    """The default wave size (1 world a wave at these batch sizes: its instance) and 8 worlds a wave (the
     packed rig State then runs the instance compiled for the rig, the headline workload's kernel)."""
     if wpw is not None:
         monkeypatch.setenv("GOI_WORLDS_PER_WAVE", wpw)
