@@ -73,8 +73,9 @@ def _carve(buf, n, dims, pitch):
 def empty_device_state(n, dims, device="cuda", pitch=None, packed=True):
     """An uninitialised device State of n worlds with capacities dims = (B, R, J, C), pitch n by default. The leaves
     are by default the consecutive parts of one buffer, which a clone copies whole; with a pitch that is a multiple of
-    64 that is the packed layout, which lets the step address every leaf from one base pointer. packed=False gives one
-    buffer per leaf, and so does code that is traced (_traced)."""
+    64 that is the packed layout, which lets the step address every leaf from one base pointer. A leaf that a program
+    keeps then keeps the State's whole buffer, and torch.save of a leaf writes all of it: keep or save a clone() of the
+    leaf. packed=False gives one buffer per leaf, and so does code that is traced (_traced)."""
     pitch = n if pitch is None else pitch
     dims = tuple(dims)
     if packed and pitch > 0 and not _traced():
@@ -131,8 +132,8 @@ def _memory_is_all(leaves):
     """Whether a copy of the leaves' memory copies all they are. A leaf that requires grad is copied as a leaf, so that its
     copy has it as its gradient's source, and so is every leaf inside a forward-mode level, where it may have a tangent,
     of a tensor subclass, which may see the copy, and in traced code."""
-    return (not _traced() and forward_ad._current_level < 0 and not any(map(_REQUIRES_GRAD, leaves))
-            and list(map(type, leaves)) == [torch.Tensor] * len(leaves))
+    return (not _traced() and forward_ad._current_level < 0 and not any(map(_REQUIRES_GRAD, _FLOATS(leaves)))
+            and list(map(type, leaves)) == _PLAIN)
 
 
 def _copy_buffer(leaves, n, dims, pitch, ptrs):
@@ -161,6 +162,8 @@ def pitch_of(state):
     return t.stride(-1) if t.dim() > 1 else t.shape[0]
 
 
+_PLAIN = [torch.Tensor] * len(wd.LEAVES)
+_FLOATS = operator.itemgetter(*[k for k, leaf in enumerate(wd.LEAVES) if np.dtype(leaf[2]) == np.float32])
 _SHAPE, _DTYPE, _DEVICE, _REQUIRES_GRAD = map(operator.attrgetter, ("shape", "dtype", "device", "requires_grad"))
 
 
