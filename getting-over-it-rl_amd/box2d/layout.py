@@ -37,7 +37,8 @@ def packed_words(dims):
 @functools.lru_cache(maxsize=64)
 def _spec(n, dims, pitch):
     """What the leaves of n worlds of capacities dims with a pitch look like, in ABI order: dtypes, shapes, strides
-    (worlds-minor), and their byte offsets as the consecutive parts of one buffer, with that buffer's bytes."""
+    (worlds-minor), and their byte offsets as the consecutive parts of one buffer, with that buffer's bytes, and the
+    offsets in elements."""
     dtypes, shapes, strides = [], [], []
     for _, _, dt, inner in wd.LEAVES:
         shape = wd.leaf_shape(inner, dims)
@@ -49,7 +50,8 @@ def _spec(n, dims, pitch):
         shapes.append((n,) + shape)
         strides.append((1, *want))
     offsets = [4 * w * pitch for w in packed_words(dims)]
-    return dtypes, shapes, strides, offsets[:-1], offsets[-1]
+    at = [o // dt.itemsize for o, dt in zip(offsets, dtypes)]
+    return dtypes, shapes, strides, offsets[:-1], offsets[-1], at
 
 
 def _traced():
@@ -61,13 +63,12 @@ def _traced():
 
 def _carve(buf, n, dims, pitch):
     """The State whose leaves are the consecutive parts of the byte buffer buf. Each leaf is a tensor of its own to autograd
-    (.data, then its shape set in place): as views of one tensor they would share its version counter and its graph, so
-    that a write into one leaf spoiled what a backward pass saved of another."""
-    dtypes, shapes, strides, offsets, _ = _spec(n, dims, pitch)
-    typed = {torch.float32: buf.view(torch.float32), torch.int32: buf.view(torch.int32), torch.bool: buf.view(torch.bool)}
-    size = {torch.float32: 4, torch.int32: 4, torch.bool: 1}
-    return wd.from_leaves([typed[dt].data.as_strided_(sh, st, off // size[dt])
-                           for dt, sh, st, off in zip(dtypes, shapes, strides, offsets)])
+    (.data, then set to its part): as views of one tensor they would share its version counter and its graph, so that a
+    write into one leaf spoiled what a backward pass saved of another."""
+    dtypes, shapes, strides, _, _, at = _spec(n, dims, pitch)
+    store = buf.untyped_storage()
+    typed = {dt: buf.view(dt) for dt in (torch.float32, torch.int32, torch.bool)}
+    return wd.from_leaves([typed[dt].data.set_(store, o, sh, st) for dt, o, sh, st in zip(dtypes, at, shapes, strides)])
 
 
 def empty_device_state(n, dims, device="cuda", pitch=None, packed=True):
@@ -142,7 +143,7 @@ def _copy_buffer(leaves, n, dims, pitch, ptrs):
     padding than worlds is copied only up to 1 MiB (16 of 65,536 rig worlds would hold 373 MB)."""
     if pitch <= 0:
         return None
-    _, _, _, offsets, nbytes = _spec(n, dims, pitch)
+    _, _, _, offsets, nbytes, _ = _spec(n, dims, pitch)
     if pitch > 2 * n and nbytes > 1 << 20:
         return None
     base = ptrs[0]
@@ -174,7 +175,7 @@ def _match(state, leaves, n, dims):
         pitch, device = state.bodies.xf_p.stride(-1), leaves[0].device
         if pitch < n:
             return None
-        dtypes, shapes, strides, _, _ = _spec(n, dims, pitch)
+        dtypes, shapes, strides, _, _, _ = _spec(n, dims, pitch)
         if (list(map(_DTYPE, leaves)) == dtypes and list(map(_SHAPE, leaves)) == shapes
                 and list(map(torch.Tensor.stride, leaves)) == strides
                 and list(map(_DEVICE, leaves)) == [device] * len(leaves)):
