@@ -1,7 +1,8 @@
 // b2_launch.hpp - the launch-side device code shared by the step's translation units: the kernel argument block
 // (Launch), the mapping of a block's lanes to worlds, the world views and the whole step of a block (step_block).
-// goi_b2.hip instantiates it for any State (leaf pointers); goi_b2_rig.hip, compiled with GOI_PACKED_STATE = 1, for
-// the 4-body rig's fixed dimensions on packed States.
+// goi_b2.hip instantiates it for any State (leaf pointers) and any worlds per wave (k_step), goi_b2_w1.hip to goi_b2_w8.hip
+// for any State at 1, 2, 4 and 8 worlds a wave (k_step_waves); goi_b2_rig.hip and goi_b2_island.hip, which define
+// GOI_PACKED_STATE 1, for the fixed dimensions of the 4-body rig and of the rig with 12 boxes on packed States.
 #pragma once
 
 #include "../../include/goi_b2.h"

@@ -42,7 +42,7 @@ struct Bodies {
 // (x - 0 * P) leaves it unchanged unless an impulse is not finite or the value is -0. A write that would change it, and
 // a separation that is NaN (the minimum over an island's rows then depends on their order), raise `changed` instead;
 // the world then runs the phase again row by row. Without either, every row saw the values it sees in Box2D's order,
-// so the results are the same floats.
+// so the results are the same floats. Run row by row, `fixed` is 0: every body is written as it comes.
 struct LaneBodies {
     Bodies bd;
     unsigned long long fixed;

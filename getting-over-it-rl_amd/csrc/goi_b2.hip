@@ -1,6 +1,6 @@
 // goi_b2.hip - the MI355X batched Box2D 2.3.1 world step (libgoi_b2.so) and its C ABI (include/goi_b2.h).
 //
-// Execution model: a step is one launch (k_step) of 64-lane wavefronts, each stepping S worlds; each world runs on a
+// Execution model: a step is one launch (k_step or an instance of it) of 64-lane wavefronts, each stepping S worlds; each world runs on a
 // group of 64 / S lanes (8 lanes at 16384 worlds) that execute its sequential code together and split its
 // independent loops (vertex, slot, body and row loops, list filters):
 //   start-of-step FindNewContacts where new_fixture, then Collide           (step.py:30-35, pairs.py:38-178)
@@ -9,8 +9,8 @@
 // goi_collide launches k_collide (the first part only). Box2D's sequential orders inside a world (contact list
 // newest first, island DFS, Gauss-Seidel sweeps, TOI events) are kept exactly; the parallelism is across worlds and
 // within the independent parts of a world's work. State leaves are read and written in place in the
-// worlds-minor layout; the solver's body arrays sit in LDS ([field][body][lane]), its constraint rows in a
-// per-block HBM scratch tile ([row][field][world]); the static terrain is a BVH over the static fixtures' fat AABBs,
+// worlds-minor layout; the solver's body arrays sit in LDS ([field][body][lane]), its constraint rows in the lanes'
+// registers or, where those do not hold them, in a per-block HBM scratch tile ([row][field][world]); the static terrain is a BVH over the static fixtures' fat AABBs,
 // shared by every world and read through L2.
 #include <algorithm>
 #include <atomic>

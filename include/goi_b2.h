@@ -342,7 +342,7 @@ int32_t goi_packed_layout(int32_t B, int32_t C, int32_t J, int32_t R, int32_t* w
  * whose workspaces do not fit a block's LDS), the blocks launched, the dynamic LDS of a block in bytes and the kernel
  * instance that ran. No counterpart in the reference: it is for tests and profiling. Returns GOI_E_ARG for a null
  * `out`; all zero before the thread's first launch. */
-#define GOI_KERNEL_GENERIC 1 /* the step for any dimensions */
+#define GOI_KERNEL_GENERIC 1 /* the step for any dimensions (an instance for the worlds per wave, or the general k_step) */
 #define GOI_KERNEL_RIG 2     /* the step compiled for the 4-body rig (5 bodies, 40 slots, 3 joints, 4 rows) */
 #define GOI_KERNEL_ISLAND 3  /* the step compiled for the rig with 12 boxes (17 bodies, 128 slots, 3 joints, 16 rows) */
 #define GOI_KERNEL_COLLIDE 4 /* goi_collide's kernel */
